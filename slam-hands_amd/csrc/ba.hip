@@ -23,10 +23,9 @@
 //                 sums the totals listed for the block (lists built on the
 //                 host; fixed order, no atomics), then S_ii += ep + lm*S_ii.
 //   k_ba_solve_*  fp64 factorization and solve, dx rounded to fp32,
-//                 retraction of the poses [t0, t1): Cholesky in one
-//                 wavefront with S in registers up to 10 free poses, LDL^T in
-//                 one workgroup with S in LDS up to 120x120, else Cholesky
-//                 blocked over many workgroups in global memory.
+//                 retraction of the poses [t0, t1): LDL^T in one workgroup up
+//                 to 120x120 (in registers up to 64x64, else in LDS), else
+//                 block LDL^T over many workgroups (k_blk_*).
 //   k_ba_backsub  grid (pixel chunk, keyframe): dz = Q (w - E^T dx),
 //                 disps += dz.
 // Host work per iteration is limited to comparing the edge list with the
@@ -516,7 +515,7 @@ struct SolveArgs {
     const double* stot;   // [N_pu + N_E][36] Schur pair blocks / row gradients
     int N_pu, P, n, n_blk, t0, t1;
     float lm, ep;
-    double* S;      // working copy of the blocked solver [(n+1)*n]: S, then b^T
+    double* S;      // working buffer of the blocked solver (blk_doubles)
     double* S_dbg;  // [n*n] assembled system (after damping), input of the solve
     double* b_dbg;  // [n]
     double* dx_dbg; // [n]
@@ -685,78 +684,6 @@ __device__ __forceinline__ void finish_solve(const SolveArgs& A, const double* x
             for (int m = 0; m < 7; m++) A.poses_next[(k - A.t0) * 7 + m] = pn[m];
     }
 }
-
-// 1/sqrt(d) in fp64: hardware estimate + two Newton steps
-// y <- y * (1.5 - 0.5 d y^2), ~1 ulp for positive normal d.
-__device__ __forceinline__ double rsqrt_f64(double d) {
-    double y = __builtin_amdgcn_rsq(d);
-    const double h = 0.5 * d;
-    y = y * (1.5 - h * y * y);
-    y = y * (1.5 - h * y * y);
-    return y;
-}
-
-// Cholesky of an N x N SPD matrix in one wavefront's registers (N <= 64):
-// lane i holds row i in r[] and ends with row i of L in r[0..i] (entries right
-// of the diagonal receive updates too and are left unused, so no lane is ever
-// predicated off). Columns go in panels of W: inside a panel, each column's
-// pivot and its entries in the panel's later columns come by readlane; then
-// every lane publishes its W panel entries to LDS (Lp, one 8W-byte row per
-// lane) and each later column k takes the panel's W updates from one
-// broadcast read of row k. Only the panel steps are sequential; the trailing
-// reads go out together. The arithmetic is the unblocked right-looking order
-// exactly: r[k] -= L[i][j] L[k][j] for j = 0, 1, ... Same pivot test as the
-// reference (every pivot > 0 before its sqrt, ba.cuh:422). inv_diag receives
-// 1/L[lane][lane].
-template <int N, int W, int kAhead = 3>
-__device__ __forceinline__ void wave_cholesky(double (&r)[N], double (*Lp)[W], bool& ok,
-                                              double& inv_diag) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int c0 = 0; c0 < N; c0 += W) {
-        const int cw = N - c0 < W ? N - c0 : W;
-#pragma unroll
-        for (int jj = 0; jj < W; jj++) {
-            if (jj < cw) {
-                const int j = c0 + jj;
-                const double d = bcast(r[j], j);
-                ok = ok && (d > 0.0);
-                const double inv = rsqrt_f64(d);  // 1 / L_jj
-                r[j] = lane == j ? d * inv : r[j] * inv;
-                if (lane == j) inv_diag = inv;
-#pragma unroll
-                for (int kk = jj + 1; kk < W; kk++)
-                    if (kk < cw) r[c0 + kk] -= r[j] * bcast(r[j], c0 + kk);
-            }
-        }
-        if (c0 + W < N) {
-#pragma unroll
-            for (int m = 0; m < W; m++) Lp[lane][m] = r[c0 + m];
-            // rows k of the panel read kAhead columns ahead of their use, in a
-            // register ring; the scheduling barriers keep the compiler from
-            // pulling each read down next to its use
-            double Lk[kAhead + 1][W];
-#pragma unroll
-            for (int q = 0; q < kAhead; q++)
-                if (c0 + W + q < N)
-#pragma unroll
-                    for (int m = 0; m < W; m++) Lk[q][m] = Lp[c0 + W + q][m];
-#pragma unroll
-            for (int k = c0 + W; k < N; k++) {
-                const int q = k - c0 - W;
-                if (k + kAhead < N)
-#pragma unroll
-                    for (int m = 0; m < W; m++) Lk[(q + kAhead) % (kAhead + 1)][m] = Lp[k + kAhead][m];
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int m = 0; m < W; m++) r[k] -= r[c0 + m] * Lk[q % (kAhead + 1)][m];
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    }
-}
-
-constexpr int kPanelW = 8;
 
 // ---- one-workgroup panel solver (n <= kPanelN: the frontend's systems) ----
 // LDL^T of the bordered matrix [S b; b^T *] in LDS, right-looking in panels
@@ -1221,218 +1148,393 @@ __global__ __launch_bounds__(256) void k_ba_solve_small(SolveArgs A) {
     solve_small_body(A, sm);
 }
 
-// ---- blocked Cholesky over many workgroups (n > kPanelN: the backend's systems) ----
-// Right-looking, lower, on the row-major working copy A.S, which holds the
-// system in rows 0..n-1 and b^T in row n (leading dimension n): factoring the
-// bordered matrix [S b; b^T *] leaves L^-1 b in row n, so the forward solve
-// costs one more panel row. In kCB-column steps: (1) k_chol_diag factors the
-// kCB x kCB diagonal block in one wavefront's registers (lane = row,
-// wave_cholesky); (2) k_chol_panel solves the rows below it (b's row
-// included) against it, one thread per row; (3) k_chol_syrk subtracts the
-// new panel's products from the trailing lower triangle in 64 x 64 tiles,
-// one workgroup per tile. k_chol_finish then runs the backward solve
-// L^T x = z in one workgroup (O(n^2), coalesced column reads) and the
-// retraction. A failed pivot is flagged in flags[2] (cleared by k_chol_init);
-// later kernels then do nothing and k_chol_finish reports the system not
-// positive definite, as the one-workgroup solvers do.
-constexpr int kCB = 64;
+// ---- block LDL^T over many workgroups (n > kPanelN: the backend's systems) ----
+// S is cut into nb x nb blocks of 64 (the last one padded with the identity)
+// and eliminated a block column at a time on the augmented system [S | I | b],
+// one launch per column. With D_j the updated diagonal block of column j and
+// T_ij = A_ij D_j^-1 for the rows i > j below it, launch j subtracts
+//   T_ij A_kj^T from A_ik    (trailing blocks, i >= k > j),
+//   T_ij V_cj^T from V_ci^T  (the identity's columns, c < j; V_ji^T = -T_ij),
+//   T_ij b_j    from b_i,
+// and forms u_j = D_j^-1 b_j; the workgroup of the next diagonal block goes on
+// to invert it. V holds W = L^-1 by columns, so the backward solve L^T x = u
+// is no second chain of steps but one product, x = W^T u (k_blk_x), and the
+// identity's blocks fill CUs that the shrinking trailing part leaves idle.
+// A block is stored in MFMA operand order (blk_at): every load and store of a
+// block is a whole 512-byte row per wave, every product's operands and
+// results are used as they lie in registers (v_mfma_f64_16x16x4: operand A is
+// (row l % 16, k l / 16) of lane l, B (k l / 16, col l % 16), result register
+// r (row 4 r + l / 16, col l % 16)), and a step's product workgroups use no
+// LDS and no barrier.
+// What bounds it: the chain of diagonal blocks (per launch two 64^3 products
+// on one CU's fp64 MFMA, 3.4 us, and the inversion, ~12 us). At n = 1188 a
+// launch takes 22.5 us and the solve 0.48 ms; the Cholesky it replaced, three
+// launches a column (diagonal block in one wave, panel rows one per thread,
+// 64 x 64 update tiles on the vector unit) and the backward solve in one
+// workgroup, took 1.56 ms (17 + 32 + 20 us a column, 258 us backward). Every pivot of the
+// inversion is tested > 0 as the reference tests its Cholesky's (ba.cuh:422);
+// a failed one is flagged in flags[2] (rewritten by k_blk_init), the launches
+// after it do nothing and k_blk_finish reports the system not positive
+// definite.
+constexpr int kBlk = 64;
+constexpr int kBlkElems = kBlk * kBlk;
 
-__global__ __launch_bounds__(256) void k_chol_init(SolveArgs A) {
-    const size_t nn = (size_t)A.n * A.n;
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < nn + A.n;
-         t += (size_t)gridDim.x * blockDim.x)
-        A.S[t] = t < nn ? A.S_dbg[t] : A.b_dbg[t - nn];
-    if (blockIdx.x == 0 && threadIdx.x == 0) A.flags[2] = 0;
+struct BlkArgs {
+    double* a;    // lower blocks of S, blk_idx(i, k) for i >= k
+    double* v;    // blocks of (L^-1)^T, blk_idx(i, c) for i > c: column c, row i of L^-1
+    double* nd;   // [nb] -D_j^-1
+    double* b;    // [nb * 64] right-hand side, then z
+    double* u;    // [nb * 64] D_j^-1 b_j
+    double* x;    // [nb * 64] solution
+    int* flags;
+    int nb, n;
+};
+
+// blocks of a lower triangle of nb block rows
+__host__ __device__ __forceinline__ size_t blk_count(int nb) { return (size_t)nb * (nb + 1) / 2; }
+__device__ __forceinline__ size_t blk_idx(int i, int k) {
+    return (blk_count(i) + k) * kBlkElems;
+}
+// offset of a wave's element: row 16 rb + (lane % 16), column 4 s + lane / 16
+__device__ __forceinline__ int blk_at(int rb, int s, int lane) {
+    return (rb * 16 + s) * 64 + lane;
 }
 
-// The diagonal block, padded to kCB x kCB with an identity block (whose
-// Cholesky is itself), so wave_cholesky runs at its compile-time size.
-__global__ __launch_bounds__(64) void k_chol_diag(SolveArgs A, int j0) {
-    __shared__ __attribute__((aligned(16))) double Lp[64][kPanelW];
-    if (A.flags[2]) return;
-    const int n = A.n, lane = threadIdx.x;
-    const int nb = min(kCB, n - j0);
-    double* S = A.S;
-    double r[kCB];
-#pragma unroll
-    for (int m = 0; m < kCB; m++)
-        r[m] = (lane < nb && m < nb) ? S[(size_t)(j0 + lane) * n + j0 + m]
-                                     : (m == lane ? 1.0 : 0.0);
-    bool ok = true;
-    double invd = 0.0;
-    wave_cholesky<kCB, kPanelW>(r, Lp, ok, invd);
-    if (lane < nb) {
-#pragma unroll
-        for (int m = 0; m < kCB; m++)
-            if (m <= lane) S[(size_t)(j0 + lane) * n + j0 + m] = r[m];
-    }
-    if (lane == 0 && !ok) A.flags[2] = 1;
+typedef double blk_d4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ blk_d4 mfma64(double a, double b, blk_d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// rows j0 + nb <= i <= n (row n is b): x L_jj^T = S[i][j0 .. j0+nb), one
-// thread per row
-__global__ __launch_bounds__(256) void k_chol_panel(SolveArgs A, int j0) {
-    __shared__ double L[kCB][kCB + 1];
-    __shared__ double invd[kCB];
-    if (A.flags[2]) return;
-    const int n = A.n;
-    const int nb = min(kCB, n - j0);
-    double* S = A.S;
-    for (int t = threadIdx.x; t < kCB * kCB; t += blockDim.x) {
-        const int r = t / kCB, c = t - (t / kCB) * kCB;
-        L[r][c] = (r < nb && c <= r) ? S[(size_t)(j0 + r) * n + j0 + c] : 0.0;
-    }
-    __syncthreads();
-    if (threadIdx.x < kCB)
-        invd[threadIdx.x] = threadIdx.x < nb ? 1.0 / L[threadIdx.x][threadIdx.x] : 0.0;
-    __syncthreads();
-    const int i = j0 + nb + blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > n) return;
-    double* row = S + (size_t)i * n + j0;
-    double x[kCB];
+// v of lane K of this lane's row of 16
+template <int K>
+__device__ __forceinline__ double row16_bcast(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + K, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + K, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+struct BlkLds {
+    double c[2][4][256];  // the waves' blocks of the panel's columns, operand order
+    double p[2][256];     // the panel's inverse diagonal block, operand order
+    double m[16][17];     // its unit lower inverse factor
+    double y[16];         // its pivots' reciprocals
+    int bad;
+};
+
+// Step K of the elimination of a 16 x 16 block held one row per lane (the
+// four rows of 16 lanes alike): rows below K lose their multiple of row K in
+// every column but K, where the multiple's negative is kept, so columns below
+// the diagonal end as the unit lower L^-1 (its entry (i, K) starts as -f and
+// takes the same updates) and the diagonal as the pivots.
+template <int K, int... Cs>
+__device__ __forceinline__ void blk_elim_step(double (&x)[16], int i16, bool& ok, double& yv,
+                                              std::integer_sequence<int, Cs...>) {
+    const double d = row16_bcast<K>(x[K]);
+    ok = ok && d > 0.0;
+    const double y = rcp_f64(d);
+    yv = i16 == K ? y : yv;
+    const double f = i16 > K ? -(x[K] * y) : 0.0;
+    ((x[Cs] = Cs == K ? (i16 > K ? f : x[Cs])
+                      : __builtin_fma(f, row16_bcast<K>(x[Cs]), x[Cs])),
+     ...);
+}
+template <int... Ks>
+__device__ __forceinline__ void blk_elim(double (&x)[16], int i16, bool& ok, double& yv,
+                                         std::integer_sequence<int, Ks...>) {
+    (blk_elim_step<Ks>(x, i16, ok, yv, std::make_integer_sequence<int, 16>{}), ...);
+}
+
+// m (this wave's 16 rows of an SPD 64 x 64 block, operand order) becomes its
+// rows of minus the inverse: a block sweep over four 16-column panels. Per
+// panel p every wave publishes its block C of the panel's columns, wave p
+// inverts the diagonal one (P^-1 = L^-T D^-1 L^-1), and with T = C P^-1 every
+// other wave's blocks become m - T C_q^T, its panel block T, and the blocks
+// of wave p P^-1 C_q^T, -P^-1. Two barriers a panel; the buffers alternate.
+// Returns whether every pivot was positive (the same for all threads).
+__device__ __forceinline__ bool blk_invert(double (&m)[16], BlkLds& L, int wave, int lane) {
+    const int i16 = lane & 15, g = lane >> 4;
+    if (threadIdx.x == 0) L.bad = 0;
 #pragma unroll
-    for (int k = 0; k < kCB; k++) {
-        if (k < nb) {
-            double v = row[k];
+    for (int p = 0; p < 4; p++) {
+        double* c = L.c[p & 1][0];
 #pragma unroll
-            for (int m = 0; m < k; m++) v -= x[m] * L[k][m];
-            x[k] = v * invd[k];
+        for (int r = 0; r < 4; r++) c[wave * 256 + r * 64 + lane] = m[4 * p + r];
+        __syncthreads();
+        if (wave == p) {
+            double x[16], yv = 0.0;
+            bool ok = true;
+#pragma unroll
+            for (int k = 0; k < 16; k++) x[k] = c[p * 256 + (k >> 2) * 64 + (k & 3) * 16 + i16];
+            blk_elim(x, i16, ok, yv, std::make_integer_sequence<int, 16>{});
+            if (g == 0) {
+#pragma unroll
+                for (int k = 0; k < 16; k++) L.m[i16][k] = k < i16 ? x[k] : k == i16 ? 1.0 : 0.0;
+                L.y[i16] = yv;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            blk_d4 pi = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const double t = L.m[4 * s + g][i16];
+                pi = mfma64(t * L.y[4 * s + g], t, pi);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) L.p[p & 1][r * 64 + lane] = pi[r];
+            if (!ok) L.bad = 1;
+        }
+        __syncthreads();
+        double pinv[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) pinv[r] = L.p[p & 1][r * 64 + lane];
+        if (wave == p) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if (q == p) continue;
+                blk_d4 t = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int s = 0; s < 4; s++) t = mfma64(c[q * 256 + s * 64 + lane], pinv[s], t);
+#pragma unroll
+                for (int r = 0; r < 4; r++) m[4 * q + r] = t[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) m[4 * p + r] = -pinv[r];
         } else {
-            x[k] = 0.0;
-        }
-    }
+            blk_d4 t = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int k = 0; k < kCB; k++)
-        if (k < nb) row[k] = x[k];
-}
-
-// trailing S[i][k] -= sum_m L[i][j0+m] L[k][j0+m] for r0 <= k <= i <= n, k < n
-// (row n is b; the upper entries of the diagonal tiles are updated too and
-// never read), r0 = j0 + nb; one workgroup per lower 64 x 64 tile of the
-// (n + 1 - r0)-row trailing block, 4 x 4 outputs per thread.
-__global__ __launch_bounds__(256) void k_chol_syrk(SolveArgs A, int j0) {
-    __shared__ double Ai[64][kCB + 1], Bk[64][kCB + 1];
-    if (A.flags[2]) return;
-    const int n = A.n;
-    const int nb = min(kCB, n - j0);
-    const int r0 = j0 + nb;
-    // blockIdx.x -> lower tile (ti, tk), tk <= ti
-    int ti = (int)((sqrtf(8.0f * (float)blockIdx.x + 1.0f) - 1.0f) * 0.5f);
-    while (ti * (ti + 1) / 2 > (int)blockIdx.x) ti--;
-    while ((ti + 1) * (ti + 2) / 2 <= (int)blockIdx.x) ti++;
-    const int tk = (int)blockIdx.x - ti * (ti + 1) / 2;
-    const int ri = r0 + ti * 64, rk = r0 + tk * 64;
-    if (rk >= n) return;  // a column tile made only of b's row
-    double* S = A.S;
-    for (int t = threadIdx.x; t < 64 * kCB; t += blockDim.x) {
-        const int r = t / kCB, m = t - (t / kCB) * kCB;
-        Ai[r][m] = (ri + r <= n && m < nb) ? S[(size_t)(ri + r) * n + j0 + m] : 0.0;
-        Bk[r][m] = (rk + r < n && m < nb) ? S[(size_t)(rk + r) * n + j0 + m] : 0.0;
-    }
-    __syncthreads();
-    const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-    double acc[4][4] = {};
-    for (int m = 0; m < nb; m++) {
-        double a[4], b[4];
+            for (int s = 0; s < 4; s++) t = mfma64(pinv[s], m[4 * p + s], t);
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            a[u] = Ai[ty + 16 * u][m];
-            b[u] = Bk[tx + 16 * u][m];
-        }
+            for (int q = 0; q < 4; q++) {
+                if (q == p) continue;
+                blk_d4 z = {m[4 * q], m[4 * q + 1], m[4 * q + 2], m[4 * q + 3]};
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+                for (int s = 0; s < 4; s++) z = mfma64(c[q * 256 + s * 64 + lane], -t[s], z);
 #pragma unroll
-            for (int v = 0; v < 4; v++) acc[u][v] += a[u] * b[v];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int i = ri + ty + 16 * u;
-        if (i > n) continue;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int k = rk + tx + 16 * v;
-            if (k < n) S[(size_t)i * n + k] -= acc[u][v];
-        }
-    }
-}
-
-// L^T x = z with L in the lower triangle of S (leading dimension n), z -> x
-// in y (LDS), one workgroup, blocks of kCB rows from the bottom. Per block,
-// wave 0 holds the block's columns of L in registers (loaded up front, so the
-// sequential substitution only waits on readlane broadcasts), then all
-// threads subtract the block's contribution from the entries above it,
-// reading L by rows (coalesced over the threads).
-__device__ void back_solve_blocked(const double* __restrict__ S, double* y, int n) {
-    const int tid = threadIdx.x;
-    for (int j0 = ((n - 1) / kCB) * kCB; j0 >= 0; j0 -= kCB) {  // backward: L^T x = z
-        const int jb = min(kCB, n - j0);
-        if (tid < 64) {
-            // lane c holds column c of the block: L[j0+k][j0+c] for k >= c
-            const int lane = tid, lc = min(lane, jb - 1);
-            double d[kCB];
-#pragma unroll
-            for (int k = 0; k < kCB; k++) d[k] = k < jb ? S[(size_t)(j0 + k) * n + j0 + lc] : 0.0;
-            double dl = 1.0;
-#pragma unroll
-            for (int k = 0; k < kCB; k++)
-                if (k == lc) dl = d[k];
-            const double invl = 1.0 / dl;
-            double v = lane < jb ? y[j0 + lane] : 0.0;
-#pragma unroll
-            for (int k = kCB - 1; k >= 0; k--) {
-                if (k < jb) {
-                    const double xk = bcast(v * invl, k);
-                    if (lane == k) v = xk;
-                    else if (lane < k) v -= d[k] * xk;
-                }
+                for (int r = 0; r < 4; r++) m[4 * q + r] = z[r];
             }
-            if (lane < jb) y[j0 + lane] = v;
+#pragma unroll
+            for (int r = 0; r < 4; r++) m[4 * p + r] = t[r];
         }
-        __syncthreads();
-        for (int i = tid; i < j0; i += blockDim.x) {
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-            int m = 0;
-            for (; m + 4 <= jb; m += 4) {
-                s0 += S[(size_t)(j0 + m) * n + i] * y[j0 + m];
-                s1 += S[(size_t)(j0 + m + 1) * n + i] * y[j0 + m + 1];
-                s2 += S[(size_t)(j0 + m + 2) * n + i] * y[j0 + m + 2];
-                s3 += S[(size_t)(j0 + m + 3) * n + i] * y[j0 + m + 3];
-            }
-            for (; m < jb; m++) s0 += S[(size_t)(j0 + m) * n + i] * y[j0 + m];
-            y[i] -= (s0 + s1) + (s2 + s3);
-        }
-        __syncthreads();
+    }
+    return L.bad == 0;
+}
+
+// The assembled system into blocks, b padded with zeros, S with the identity;
+// workgroup 0 inverts the first diagonal block.
+__global__ __launch_bounds__(256) void k_blk_init(SolveArgs A, BlkArgs B) {
+    __shared__ BlkLds L;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i16 = lane & 15, g = lane >> 4;
+    int bi = (int)((sqrtf(8.0f * (float)blockIdx.x + 1.0f) - 1.0f) * 0.5f);
+    while (bi > 0 && blk_count(bi) > blockIdx.x) bi--;
+    while (blk_count(bi + 1) <= blockIdx.x) bi++;
+    const int bk = (int)(blockIdx.x - blk_count(bi));
+    const int n = B.n;
+    const int row = bi * kBlk + wave * 16 + i16;
+    double m[16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+        const int col = bk * kBlk + 4 * s + g;
+        // the lower triangle (a diagonal block's upper entries by symmetry)
+        const int hi = max(row, col), lo = min(row, col);
+        const double t = A.S_dbg[(size_t)min(hi, n - 1) * n + min(lo, n - 1)];
+        m[s] = hi < n ? t : row == col ? 1.0 : 0.0;
+    }
+    double* a = B.a + (size_t)blockIdx.x * kBlkElems;
+#pragma unroll
+    for (int s = 0; s < 16; s++) a[blk_at(wave, s, lane)] = m[s];
+    if (bi == bk && threadIdx.x < kBlk) {
+        const int k = bi * kBlk + threadIdx.x;
+        B.b[k] = k < n ? A.b_dbg[k] : 0.0;
+    }
+    if (blockIdx.x == 0) {
+        const bool ok = blk_invert(m, L, wave, lane);
+#pragma unroll
+        for (int s = 0; s < 16; s++) B.nd[blk_at(wave, s, lane)] = m[s];
+        if (threadIdx.x == 0) B.flags[2] = ok ? 0 : 1;
     }
 }
 
-constexpr int kFinishWG = 512;
-__global__ __launch_bounds__(kFinishWG) void k_chol_finish(SolveArgs A) {
-    extern __shared__ double smem[];
-    const int n = A.n;
-    double* b = smem;
-    const bool ok = A.flags[2] == 0;
-    const int halt_word = solve_halt_word(A);
-    for (int t = threadIdx.x; t < n; t += blockDim.x) b[t] = A.S[(size_t)n * n + t];  // z
-    __syncthreads();
-    if (ok) back_solve_blocked(A.S, b, n);
-    __syncthreads();
-    finish_solve(A, b, ok, halt_word, A.poses + 7 * A.t0);
+// Launch j of the elimination (see above): the trailing blocks (the next
+// diagonal one first), then the identity's blocks of rows j + 1 .. nb - 1,
+// columns 0 .. j, then one workgroup for u_j.
+__global__ __launch_bounds__(256) void k_blk_step(BlkArgs B, int j) {
+    __shared__ BlkLds L;
+    if (B.flags[2]) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i16 = lane & 15, g = lane >> 4;
+    const int R = B.nb - 1 - j;
+    const int ntrail = R * (R + 1) / 2;
+    const double* nd = B.nd + (size_t)j * kBlkElems;
+    const double* bj = B.b + j * kBlk;
+    const int id = blockIdx.x;
+    if (id == ntrail + R * (j + 1)) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 16; k++) s -= nd[blk_at(wave, k, lane)] * bj[4 * k + g];
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        if (g == 0) B.u[j * kBlk + wave * 16 + i16] = s;
+        return;
+    }
+    const bool trail = id < ntrail;
+    int i, k;
+    if (trail) {
+        int t = (int)((sqrtf(8.0f * (float)id + 1.0f) - 1.0f) * 0.5f);
+        while (t > 0 && (int)blk_count(t) > id) t--;
+        while ((int)blk_count(t + 1) <= id) t++;
+        i = j + 1 + t;
+        k = j + 1 + id - (int)blk_count(t);
+    } else {
+        const int t = (id - ntrail) / (j + 1);
+        i = j + 1 + t;
+        k = id - ntrail - t * (j + 1);
+    }
+    // this wave's 16 rows of A_ij, and -D_j^-1
+    const double* aij = B.a + blk_idx(i, j);
+    double a[16], d[4][16];
+#pragma unroll
+    for (int s = 0; s < 16; s++) a[s] = aij[blk_at(wave, s, lane)];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int s = 0; s < 16; s++) d[t][s] = nd[blk_at(t, s, lane)];
+    const blk_d4 zero = {0.0, 0.0, 0.0, 0.0};
+    if (!trail && k == j) {
+        // -T_ij by rows i: it is the transposed block of the identity's column j
+        blk_d4 t4[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) t4[t] = zero;
+#pragma unroll
+        for (int s = 0; s < 16; s++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) t4[t] = mfma64(a[s], d[t][s], t4[t]);
+        double* v = B.v + blk_idx(i, j);
+        double db[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const double bk = bj[16 * t + i16];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                v[blk_at(t, 4 * wave + r, lane)] = t4[t][r];
+                db[r] += t4[t][r] * bk;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) db[r] += __shfl_xor(db[r], o, 64);
+            if (i16 == 0) B.b[i * kBlk + wave * 16 + 4 * r + g] += db[r];
+        }
+        return;
+    }
+    // the block to update and the second factor (A_kj by rows, or V_cj)
+    double* out = trail ? B.a + blk_idx(i, k) : B.v + blk_idx(i, k);
+    const double* fac = trail ? B.a + blk_idx(k, j) : B.v + blk_idx(j, k);
+    blk_d4 acc[4], t4[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            acc[t][r] = out[trail ? blk_at(wave, 4 * t + r, lane) : blk_at(t, 4 * wave + r, lane)];
+    // -T_ij^T: columns are this wave's rows i, so a result register is the
+    // next product's operand
+#pragma unroll
+    for (int t = 0; t < 4; t++) t4[t] = zero;
+#pragma unroll
+    for (int s = 0; s < 16; s++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) t4[t] = mfma64(d[t][s], a[s], t4[t]);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int s = 0; s < 16; s++) d[t][s] = fac[blk_at(t, s, lane)];
+    if (trail) {
+#pragma unroll
+        for (int s = 0; s < 16; s++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc[t] = mfma64(d[t][s], t4[s >> 2][s & 3], acc[t]);
+    } else {
+#pragma unroll
+        for (int s = 0; s < 16; s++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) acc[t] = mfma64(t4[s >> 2][s & 3], d[t][s], acc[t]);
+    }
+    if (id == 0) {  // the next diagonal block
+        double m[16];
+#pragma unroll
+        for (int s = 0; s < 16; s++) m[s] = acc[s >> 2][s & 3];
+        const bool ok = blk_invert(m, L, wave, lane);
+        double* ndn = B.nd + (size_t)(j + 1) * kBlkElems;
+#pragma unroll
+        for (int s = 0; s < 16; s++) ndn[blk_at(wave, s, lane)] = m[s];
+        if (threadIdx.x == 0 && !ok) B.flags[2] = 1;
+        return;  // the block itself is not read again
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            out[trail ? blk_at(wave, 4 * t + r, lane) : blk_at(t, 4 * wave + r, lane)] = acc[t][r];
+}
+
+// x_c = u_c + sum_{i > c} V_ci^T u_i, one workgroup per block column.
+__global__ __launch_bounds__(256) void k_blk_x(BlkArgs B) {
+    if (B.flags[2]) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i16 = lane & 15, g = lane >> 4;
+    const int c = blockIdx.x;
+    double s = 0.0;
+#pragma unroll 2
+    for (int i = c + 1; i < B.nb; i++) {
+        const double* v = B.v + blk_idx(i, c);
+        const double* u = B.u + i * kBlk;
+        double e[16], w[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) e[k] = v[blk_at(wave, k, lane)];
+#pragma unroll
+        for (int k = 0; k < 16; k++) w[k] = u[4 * k + g];
+#pragma unroll
+        for (int k = 0; k < 16; k++) s += e[k] * w[k];
+    }
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    const int row = c * kBlk + wave * 16 + i16;
+    if (g == 0) B.x[row] = s + B.u[row];
+}
+
+__global__ __launch_bounds__(256) void k_blk_finish(SolveArgs A, BlkArgs B) {
+    finish_solve(A, B.x, B.flags[2] == 0, solve_halt_word(A), A.poses + 7 * A.t0);
+}
+
+// doubles of a solve's working buffer: blocks of S and of L^-1, the diagonal
+// inverses, b, u and x
+size_t blk_doubles(int n) {
+    const int nb = (n + kBlk - 1) / kBlk;
+    return (2 * blk_count(nb) + nb) * kBlkElems + 3 * (size_t)nb * kBlk;
 }
 
 int solve_blocked(const SolveArgs& A, hipStream_t stream) {
-    const int n = A.n;
-    hipLaunchKernelGGL(k_chol_init, dim3(std::min(1024, (n * (n + 1) + 255) / 256)), dim3(256),
-                       0, stream, A);
-    for (int j0 = 0; j0 < n; j0 += kCB) {
-        hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(64), 0, stream, A, j0);
-        const int rows = n + 1 - std::min(n, j0 + kCB);  // trailing rows, b's included
-        hipLaunchKernelGGL(k_chol_panel, dim3((rows + 255) / 256), dim3(256), 0, stream, A, j0);
-        if (rows <= 1) break;
-        const int T = (rows + 63) / 64;
-        hipLaunchKernelGGL(k_chol_syrk, dim3(T * (T + 1) / 2), dim3(256), 0, stream, A, j0);
+    const int nb = (A.n + kBlk - 1) / kBlk;
+    BlkArgs B;
+    B.n = A.n;
+    B.nb = nb;
+    B.flags = A.flags;
+    B.a = A.S;
+    B.v = B.a + blk_count(nb) * kBlkElems;
+    B.nd = B.v + blk_count(nb) * kBlkElems;
+    B.b = B.nd + (size_t)nb * kBlkElems;
+    B.u = B.b + (size_t)nb * kBlk;
+    B.x = B.u + (size_t)nb * kBlk;
+    hipLaunchKernelGGL(k_blk_init, dim3((unsigned)blk_count(nb)), dim3(256), 0, stream, A, B);
+    for (int j = 0; j < nb; j++) {
+        const int R = nb - 1 - j;
+        hipLaunchKernelGGL(k_blk_step, dim3(R * (R + 1) / 2 + R * (j + 1) + 1), dim3(256), 0,
+                           stream, B, j);
     }
-    hipLaunchKernelGGL(k_chol_finish, dim3(1), dim3(kFinishWG), (size_t)n * sizeof(double),
-                       stream, A);
+    hipLaunchKernelGGL(k_blk_x, dim3(nb), dim3(256), 0, stream, B);
+    hipLaunchKernelGGL(k_blk_finish, dim3(1), dim3(256), 0, stream, A, B);
     SLK_HIP(hipGetLastError());
     return SLK_OK;
 }
@@ -2822,7 +2924,7 @@ int ba_prepare(slk_ctx* ctx, const IterArgs& I, const int* ii_host, const int* j
         SLK_TRY(s->Q.ensure((size_t)s->N_kf * HW * sizeof(double)));
         SLK_TRY(s->Wv.ensure((size_t)s->N_kf * HW * sizeof(double)));
     }
-    if (n > (size_t)kPanelN) SLK_TRY(s->S.ensure((n + 1) * n * sizeof(double)));
+    if (n > (size_t)kPanelN) SLK_TRY(s->S.ensure(blk_doubles(s->n) * sizeof(double)));
     SLK_TRY(s->S_dbg.ensure(n * n * sizeof(double)));
     SLK_TRY(s->b_dbg.ensure(n * sizeof(double)));
     SLK_TRY(s->dx_dbg.ensure(n * sizeof(double)));
