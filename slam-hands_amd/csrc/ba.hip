@@ -6,7 +6,7 @@
 // accum, damping_Q, EEt6x6, Ev6x1, EvT6x1, depth_update, and the host
 // orchestration BundleAdjustment::iterate) with se3.cuh for the geometry.
 //
-// Iteration = 5 kernels on one stream:
+// Iteration = 6 kernels on one stream:
 //   k_ba_lin_*    grid (pixel chunk, keyframe): every edge whose depth owner
 //                 (ii) is that keyframe is linearized for the chunk's pixels in
 //                 fp64. Per edge and chunk only Hjj (21) and vj (6) are
@@ -15,10 +15,10 @@
 //                 Q = 1/(C + 0.2 eta + 1e-7) and the E rows of the keyframe
 //                 are accumulated in place, so the per-edge Eii/Eij/Cii/bz
 //                 arrays of the reference never exist.
-//   k_ba_schur    one workgroup per item over all pixels: E_r1 Q E_r2^T for
-//                 the upper pairs of E rows sharing a keyframe, E_r Q w per
-//                 row; then one workgroup per edge sums its chunk partials and
-//                 expands them to the four blocks with the edge's Adj.
+//   k_ba_etot     one wave per edge sums its chunk partials and expands them
+//                 to the four blocks with the edge's Adj.
+//   k_ba_schur    [E; w] Q [E; w]^T per keyframe on fp64 MFMA: the blocks of
+//                 its pairs of E rows and E_r Q w per row.
 //   k_ba_assemble one workgroup per 6x6 block of S and per 6 entries of b:
 //                 sums the totals listed for the block (lists built on the
 //                 host; fixed order, no atomics), then S_ii += ep + lm*S_ii.
@@ -31,6 +31,7 @@
 // Host work per iteration is limited to comparing the edge list with the
 // cached one; index structures are rebuilt and uploaded only when it changes.
 #include <algorithm>
+#include <array>
 #include <cstring>
 #include <map>
 #include <utility>
@@ -45,7 +46,6 @@ namespace {
 
 constexpr int kLinWG = 256;
 constexpr int kLinPx = 256;  // pixels per linearization workgroup (<= kLinWG, a multiple of 64)
-constexpr int kSchWG = 256;
 constexpr int kNH = 90;      // 78 upper-triangle Hessian entries + vi(6) + vj(6)
 // Per (edge, pixel chunk) the linearization reduces only Hjj = sum w Jj Jj^T
 // (21 upper entries) and vj = sum w r Jj (6): Ji = -Adj(Tij) Jj per pixel
@@ -71,7 +71,8 @@ struct PlanDev {
     const int* row_kf;    // [N_E] compact kf
     const int* kf_rptr;   // [N_kf+1]
     const int* kf_rows;   // [N_E]
-    const int* pairs;     // [N_pu][3] = r1, r2, kc (r1 <= r2)
+    const int* zitems;    // [..][3] = compact kf, first row tile, first column tile (k_ba_schur)
+    const int* kf_pbase;  // [N_kf] first row pair of each kf
     const int* sblk;      // [n_blk] a*P + b
     const int* sblk_ptr;  // [n_blk+1]
     const int* sblk_src;  // contributions (see encode_*)
@@ -79,7 +80,7 @@ struct PlanDev {
     const int* bv_src;
     const int* blkmap;    // [P*P] block id of (a, b) in sblk, or -1
 };
-constexpr int kPlanParts = 16;
+constexpr int kPlanParts = 17;
 
 // contribution codes: type in bits 30..31
 __host__ __device__ __forceinline__ int code(int type, int v) { return (type << 30) | v; }
@@ -232,6 +233,17 @@ __device__ void edge_totals(int e, const float* __restrict__ poses, const int* _
     }
 }
 
+// one wave per edge
+__global__ __launch_bounds__(64) void k_ba_etot(const float* __restrict__ poses,
+                                                const int* __restrict__ ii,
+                                                const int* __restrict__ jj,
+                                                const double* __restrict__ hpart,
+                                                double* __restrict__ etot, int nch) {
+    __shared__ double sh[kNJ + 72];
+    const int e = blockIdx.x;
+    edge_totals(e, poses, ii, jj, hpart, etot + (size_t)e * kNT, nch, sh);
+}
+
 // ------------------------------------------------------- k_ba_lin_kf ----
 // Edge-serial linearization (a keyframe with two edges to one free pose):
 // grid (pixel chunk, keyframe), the workgroup walks the keyframe's edges in
@@ -241,7 +253,8 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_kf(
     const float* __restrict__ poses, const float* __restrict__ disps,
     const float* __restrict__ intr, const int* __restrict__ ii, const int* __restrict__ jj,
     const float* __restrict__ eta, double* __restrict__ hpart, double* __restrict__ E,
-    double* __restrict__ Qo, double* __restrict__ Wo, int HW, int W, int nch, int motion_only) {
+    double* __restrict__ Qo, double* __restrict__ Wo, int HW, int HWs, int W, int nch,
+    int motion_only) {
     __shared__ double red[kNJ * (kLinWG / 64)];
     __shared__ double rel[7];
     const int chunk = blockIdx.x;
@@ -250,11 +263,13 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_kf(
     const double fx = intr[0], fy = intr[1], cx = intr[2], cy = intr[3];
     const int k = chunk * kLinPx + threadIdx.x;
     const bool vpx = (int)threadIdx.x < kLinPx && k < HW;  // threads past the chunk idle
+    // E, Q and w have rows of HWs >= HW pixels whose end stays zero
+    const bool spx = (int)threadIdx.x < kLinPx && k < HWs;
     const int r0 = plan.kf_rptr[kc], r1 = plan.kf_rptr[kc + 1];
-    if (!motion_only && vpx) {
+    if (!motion_only && spx) {
         for (int r = r0; r < r1; r++) {
-            double* er = E + (size_t)plan.kf_rows[r] * 6 * HW;
-            for (int n = 0; n < 6; n++) er[(size_t)n * HW + k] = 0.0;
+            double* er = E + (size_t)plan.kf_rows[r] * 6 * HWs;
+            for (int n = 0; n < 6; n++) er[(size_t)n * HWs + k] = 0.0;
         }
     }
     double Cacc = 0.0, Wacc = 0.0;
@@ -293,24 +308,24 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_kf(
                 if (ri >= 0) {  // Ji-row contribution -Adj g (ba.cuh:139-140)
                     double gi[6];
                     adj_se3(tij, qij, g, gi);
-                    double* er = E + (size_t)ri * 6 * HW + k;
+                    double* er = E + (size_t)ri * 6 * HWs + k;
 #pragma unroll
-                    for (int n = 0; n < 6; n++) er[(size_t)n * HW] -= gi[n];
+                    for (int n = 0; n < 6; n++) er[(size_t)n * HWs] -= gi[n];
                 }
                 if (rj >= 0) {
-                    double* er = E + (size_t)rj * 6 * HW + k;
+                    double* er = E + (size_t)rj * 6 * HWs + k;
 #pragma unroll
-                    for (int n = 0; n < 6; n++) er[(size_t)n * HW] += g[n];
+                    for (int n = 0; n < 6; n++) er[(size_t)n * HWs] += g[n];
                 }
             }
         }
         block_sum_to(acc, red, hpart + ((size_t)e * nch + chunk) * kNJ);
     }
-    if (!motion_only && vpx) {
+    if (!motion_only && spx) {
         // damping_Q_kernel with ep = 1e-7 (ba.cuh:266-281, 701-702)
-        const double c = Cacc + 0.2 * (double)eta[(size_t)kf * HW + k] + 1e-7;
-        Qo[(size_t)kc * HW + k] = 1.0 / c;
-        Wo[(size_t)kc * HW + k] = Wacc;
+        const double c = vpx ? Cacc + 0.2 * (double)eta[(size_t)kf * HW + k] + 1e-7 : 1.0;
+        Qo[(size_t)kc * HWs + k] = vpx ? 1.0 / c : 0.0;
+        Wo[(size_t)kc * HWs + k] = Wacc;
     }
 }
 
@@ -330,7 +345,8 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_wv(
     const float* __restrict__ poses, const float* __restrict__ disps,
     const float* __restrict__ intr, const int* __restrict__ ii, const int* __restrict__ jj,
     const float* __restrict__ eta, double* __restrict__ hpart, double* __restrict__ E,
-    double* __restrict__ Qo, double* __restrict__ Wo, int HW, int W, int nch, int motion_only) {
+    double* __restrict__ Qo, double* __restrict__ Wo, int HW, int HWs, int W, int nch,
+    int motion_only) {
     __shared__ double eri_s[kLinWaves][6][kLinPx];  // keyframe-pose E row, per wave
     __shared__ double cw_s[kLinWaves][2][kLinPx];   // C and w, per wave
     const int chunk = blockIdx.x;
@@ -378,8 +394,13 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_wv(
         for (int n = 0; n < kNJ; n++) acc[n] = 0.0;
 #pragma unroll
         for (int s = 0; s < kLinPPL; s++) {
-            if (!vpx[s]) continue;
             const int k = kpx[s], px = s * 64 + lane;
+            if (!vpx[s]) {
+                // E, Q and w have rows of HWs >= HW pixels whose end stays zero
+                if (!motion_only && !stereo && rj >= 0 && k < HWs)
+                    for (int n = 0; n < 6; n++) E[((size_t)rj * 6 + n) * HWs + k] = 0.0;
+                continue;
+            }
             Lin L;
             lin_pixel(tij, qij, fx, fy, cx, cy, k, W, dsp[s], (double)tgu[s], (double)tgv[s],
                       (double)wtu[s], (double)wtv[s], L);
@@ -399,9 +420,9 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_wv(
                         for (int n = 0; n < 6; n++) eri_s[wave][n][px] -= gi[n];
                     }
                     if (rj >= 0) {
-                        double* er = E + (size_t)rj * 6 * HW + k;
+                        double* er = E + (size_t)rj * 6 * HWs + k;
 #pragma unroll
-                        for (int n = 0; n < 6; n++) er[(size_t)n * HW] = g[n];
+                        for (int n = 0; n < 6; n++) er[(size_t)n * HWs] = g[n];
                     }
                 }
             }
@@ -417,7 +438,7 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_wv(
     if (!motion_only) {
         // one pixel per thread: the per-wave slices in wave order
         const int px = threadIdx.x, k = chunk * kLinPx + px;
-        if (px < kLinPx && k < HW) {
+        if (px < kLinPx && k < HWs) {
             double c = 0.0, w = 0.0;
 #pragma unroll
             for (int v = 0; v < kLinWaves; v++) {
@@ -425,18 +446,19 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_wv(
                 w += cw_s[v][1][px];
             }
             // damping_Q_kernel with ep = 1e-7 (ba.cuh:266-281, 701-702)
-            Qo[(size_t)kc * HW + k] = 1.0 / (c + 0.2 * (double)eta[(size_t)kf * HW + k] + 1e-7);
-            Wo[(size_t)kc * HW + k] = w;
+            const double e = k < HW ? 0.2 * (double)eta[(size_t)kf * HW + k] : 0.0;
+            Qo[(size_t)kc * HWs + k] = k < HW ? 1.0 / (c + e + 1e-7) : 0.0;
+            Wo[(size_t)kc * HWs + k] = w;
             // the keyframe's own pose row
             const int ri = e1 > e0 ? plan.edge_ri[plan.kf_eidx[e0]] : -1;
             if (ri >= 0) {
-                double* er = E + (size_t)ri * 6 * HW + k;
+                double* er = E + (size_t)ri * 6 * HWs + k;
 #pragma unroll
                 for (int n = 0; n < 6; n++) {
                     double t = 0.0;
 #pragma unroll
                     for (int v = 0; v < kLinWaves; v++) t += eri_s[v][n][px];
-                    er[(size_t)n * HW] = t;
+                    er[(size_t)n * HWs] = t;
                 }
             }
         }
@@ -444,63 +466,181 @@ __global__ __launch_bounds__(kLinWG) void k_ba_lin_wv(
 }
 
 // -------------------------------------------------------- k_ba_schur ----
-// One workgroup per item over all pixels: E_r1 Q E_r2^T for an upper pair of
-// E rows sharing a keyframe (EEt6x6_kernel, ba.cuh:303-342), or E_r Q w for a
-// row (Ev6x1_kernel, ba.cuh:346-372); the 36 (or 6) totals go to stot[item].
-// Workgroups past the N_items Schur items each form one edge's totals
-// (edge_totals, wave 0), which need only the linearization's partials.
-__global__ __launch_bounds__(kSchWG) void k_ba_schur(PlanDev plan, const double* __restrict__ E,
-                                                     const double* __restrict__ Q,
-                                                     const double* __restrict__ Wv,
-                                                     double* __restrict__ stot, int HW,
-                                                     int N_pu, int N_items,
-                                                     const float* __restrict__ poses,
-                                                     const int* __restrict__ ii,
-                                                     const int* __restrict__ jj,
-                                                     const double* __restrict__ hpart,
-                                                     double* __restrict__ etot, int nch) {
-    __shared__ double red[36 * (kSchWG / 64)];
-    const int item = blockIdx.x;
-    if (item >= N_items) {
-        if (threadIdx.x < 64)
-            edge_totals(item - N_items, poses, ii, jj, hpart,
-                        etot + (size_t)(item - N_items) * kNT, nch, red);
-        return;
-    }
-    double acc[36];
+// Z = [E; w] Q [E; w]^T of a keyframe over its pixels, whose blocks are the
+// reference's E_r1 Q E_r2^T of the row pairs (EEt6x6_kernel, ba.cuh:303-342)
+// and E_r Q w of the rows (Ev6x1_kernel, ba.cuh:346-372), in 16 x 16 tiles on
+// v_mfma_f64_16x16x4. An item is the upper tiles of one group of kSchT row
+// tiles (13 E rows and w), or a group's tiles with kSchTB column tiles right
+// of it; a workgroup is an item over one of nsp shares of the pixels, split
+// again over its four waves.
+// Lane l takes row l % 16 of a tile and, of each 16 pixels, 2 (l / 16), the
+// next one and the two 8 further, as two 16-byte loads (a row's four lanes read
+// 64 bytes at a time): the four MFMA steps of 16 pixels take the pixels in that
+// order on both operands, so a product reads each E row once, in whole cache
+// lines, straight into operands. The next 16 pixels are in flight during the
+// current ones' products. The waves' tiles are added in wave order in LDS, and the pair blocks and row gradients of the share go to
+// stot[share][item][36]; the assembly adds the shares in order.
+// What bounds it: reading E (324 MB for the 200-keyframe, 2000-edge graph at
+// 48x64, 65 us at the card's copy rate) and the fp64 MFMAs (60 us with the
+// padding to 16); it takes 120 us (two waves a SIMD: 175 us at one, with all
+// operands in registers). One workgroup per row pair on the vector unit read
+// every E row once per pair, 3.9 GB from L2, in 401 us.
+constexpr int kSchT = 5;
+constexpr int kSchTB = 3;  // column tiles of an item between two groups
+
+typedef double sch_d4 __attribute__((ext_vector_type(4)));
+
+struct SchurArgs {
+    PlanDev plan;
+    const double* E;
+    const double* Q;
+    const double* Wv;
+    double* stot;
+    int HWs;             // row stride of E, Q, Wv: h*w rounded up to 16, zero-filled
+    int N_pu;            // row pairs
+    int nsp;             // pixel shares
+    size_t share;        // doubles of stot per share
+};
+
+// rows 16 t + l % 16 of a keyframe: its E rows (6 each), then w
+struct SchurRow {
+    const double* p;
+    bool in;
+};
+__device__ __forceinline__ SchurRow schur_row(const SchurArgs& A, int kc, int r0, int nr, int R) {
+    SchurRow s;
+    s.in = R <= 6 * nr;
+    if (R < 6 * nr)
+        s.p = A.E + ((size_t)A.plan.kf_rows[r0 + R / 6] * 6 + R % 6) * A.HWs;
+    else
+        s.p = A.Wv + (size_t)kc * A.HWs;
+    return s;
+}
+
+// TA x TB tiles of rows 16 ta0.. and columns 16 tb0..; on the diagonal
+// (kDiag, ta0 == tb0, TA == TB) the upper tiles.
+template <int TA, int TB, bool kDiag>
+__device__ __forceinline__ void schur_item(const SchurArgs& A, int kc, int ta0, int tb0, int share,
+                                           double* lds) {
+    constexpr int NT = kDiag ? TA * (TA + 1) / 2 : TA * TB;
+    constexpr int NB = kDiag ? 0 : TB;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int i16 = lane & 15, lg = lane >> 4;
+    const int r0 = A.plan.kf_rptr[kc], nr = A.plan.kf_rptr[kc + 1] - r0;
+    SchurRow ra[TA], rb[NB + 1];
 #pragma unroll
-    for (int n = 0; n < 36; n++) acc[n] = 0.0;
-    if (item < N_pu) {
-        const int r1 = plan.pairs[item * 3 + 0], r2 = plan.pairs[item * 3 + 1];
-        const int kc = plan.pairs[item * 3 + 2];
-        const double* e1 = E + (size_t)r1 * 6 * HW;
-        const double* e2 = E + (size_t)r2 * 6 * HW;
-        const double* qk = Q + (size_t)kc * HW;
-        for (int k = threadIdx.x; k < HW; k += kSchWG) {
-            const double q = qk[k];
-            double a[6], b[6];
+    for (int t = 0; t < TA; t++) ra[t] = schur_row(A, kc, r0, nr, 16 * (ta0 + t) + i16);
 #pragma unroll
-            for (int n = 0; n < 6; n++) {
-                a[n] = e1[(size_t)n * HW + k] * q;
-                b[n] = e2[(size_t)n * HW + k];
+    for (int t = 0; t < NB; t++) rb[t] = schur_row(A, kc, r0, nr, 16 * (tb0 + t) + i16);
+    const double* qp = A.Q + (size_t)kc * A.HWs;
+    sch_d4 z[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) z[t] = sch_d4{0.0, 0.0, 0.0, 0.0};
+    const int G = A.HWs / 16, W = A.nsp * 4, me = share * 4 + wave;
+    const int g0 = (int)((long)G * me / W), g1 = (int)((long)G * (me + 1) / W);
+    double2 va[TA][2], vb[NB + 1][2], vq[2];
+    auto load = [&](int g) {
+        const int k = g * 16 + 2 * lg;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            vq[h] = *(const double2*)(qp + k + 8 * h);
+#pragma unroll
+            for (int t = 0; t < TA; t++) va[t][h] = *(const double2*)(ra[t].p + k + 8 * h);
+#pragma unroll
+            for (int t = 0; t < NB; t++) vb[t][h] = *(const double2*)(rb[t].p + k + 8 * h);
+        }
+    };
+    if (g0 < g1) load(g0);
+    for (int g = g0; g < g1; g++) {
+        double a[TA][4], b[kDiag ? TA : TB][4], q[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) q[s] = s & 1 ? vq[s >> 1].y : vq[s >> 1].x;
+#pragma unroll
+        for (int t = 0; t < TA; t++)
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                a[t][s] = ra[t].in ? (s & 1 ? va[t][s >> 1].y : va[t][s >> 1].x) : 0.0;
+#pragma unroll
+        for (int t = 0; t < (kDiag ? TA : TB); t++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                if constexpr (kDiag)
+                    b[t][s] = a[t][s] * q[s];
+                else
+                    b[t][s] = rb[t].in ? (s & 1 ? vb[t][s >> 1].y : vb[t][s >> 1].x) * q[s] : 0.0;
             }
+        if (g + 1 < g1) load(g + 1);
 #pragma unroll
-            for (int n = 0; n < 6; n++)
+        for (int s = 0; s < 4; s++) {
+            int tt = 0;
 #pragma unroll
-                for (int m = 0; m < 6; m++) acc[n * 6 + m] += a[n] * b[m];
+            for (int ta = 0; ta < TA; ta++)
+#pragma unroll
+                for (int tb = kDiag ? ta : 0; tb < (kDiag ? TA : TB); tb++, tt++)
+                    z[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ta][s], b[tb][s], z[tt], 0, 0, 0);
+        }
+    }
+    // the waves' tiles added in LDS in turn
+    for (int v = 0; v < 4; v++) {
+        if (wave == v) {
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    double* l = lds + (t * 4 + r) * 64 + lane;
+                    *l = v > 0 ? *l + z[t][r] : z[t][r];
+                }
+        }
+        __syncthreads();
+    }
+    // entry (4 r + l / 16, l % 16) of tile tt, one thread per (r, l): into the
+    // pair blocks (pair (a, b) of the keyframe's rows is pb + a nr -
+    // a (a - 1) / 2 + b - a) and, from w's column, the row gradients
+    double* out = A.stot + share * A.share;
+    const int pb = A.plan.kf_pbase[kc];
+    int tt = 0;
+    for (int ta = 0; ta < TA; ta++)
+        for (int tb = kDiag ? ta : 0; tb < (kDiag ? TA : TB); tb++, tt++) {
+            const double t = lds[tt * 256 + threadIdx.x];
+            const int R = 16 * (ta0 + ta) + 4 * wave + lg, Cc = 16 * (tb0 + tb) + i16;
+            const int pa = R / 6, n = R - 6 * pa, pc = Cc / 6, m = Cc - 6 * pc;
+            if (pa >= nr || pa > pc) continue;
+            if (pc < nr) {
+                double* o = out + (size_t)(pb + pa * nr - pa * (pa - 1) / 2 + pc - pa) * 36;
+                o[n * 6 + m] = t;
+                // a pair block (a, a) cut by a tile border: its other half
+                if (pa == pc && R / 16 != Cc / 16) o[m * 6 + n] = t;
+            } else if (Cc == 6 * nr) {
+                out[(size_t)(A.N_pu + A.plan.kf_rows[r0 + pa]) * 36 + n] = t;
+            }
+        }
+}
+
+__global__ __launch_bounds__(256, 2) void k_ba_schur(SchurArgs A) {
+    __shared__ double lds[kSchT * kSchTB * 256];
+    const int item = blockIdx.x / A.nsp, share = blockIdx.x - item * A.nsp;
+    const int* it = A.plan.zitems + 3 * item;
+    const int kc = it[0], ta0 = it[1], tb0 = it[2];
+    const int nr = A.plan.kf_rptr[kc + 1] - A.plan.kf_rptr[kc];
+    const int tb = (6 * nr + 16) / 16 - tb0;  // column tiles from the item's first on
+    if (ta0 == tb0) {
+        switch (tb) {
+            case 1: schur_item<1, 1, true>(A, kc, ta0, tb0, share, lds); break;
+            case 2: schur_item<2, 2, true>(A, kc, ta0, tb0, share, lds); break;
+            case 3: schur_item<3, 3, true>(A, kc, ta0, tb0, share, lds); break;
+            case 4: schur_item<4, 4, true>(A, kc, ta0, tb0, share, lds); break;
+            default: schur_item<kSchT, kSchT, true>(A, kc, ta0, tb0, share, lds); break;
         }
     } else {
-        const int r = item - N_pu;
-        const int kc = plan.row_kf[r];
-        const double* er = E + (size_t)r * 6 * HW;
-        for (int k = threadIdx.x; k < HW; k += kSchWG) {
-            const double qw = Q[(size_t)kc * HW + k] * Wv[(size_t)kc * HW + k];
-#pragma unroll
-            for (int n = 0; n < 6; n++) acc[n] += qw * er[(size_t)n * HW + k];
+        switch (tb) {
+            case 1: schur_item<kSchT, 1, false>(A, kc, ta0, tb0, share, lds); break;
+            case 2: schur_item<kSchT, 2, false>(A, kc, ta0, tb0, share, lds); break;
+            default: schur_item<kSchT, kSchTB, false>(A, kc, ta0, tb0, share, lds); break;
         }
     }
-    block_sum_to(acc, red, stot + (size_t)item * 36);
 }
+static_assert(kSchT == 5 && kSchTB == 3 && kSchT * (kSchT + 1) / 2 <= kSchT * kSchTB,
+              "the cases of k_ba_schur and its LDS");
 
 // ----------------------------------------------------------- solve ------
 // the BA status words (BaState::flags): [0] the last step was rejected, [1]
@@ -512,7 +652,9 @@ constexpr int kBaFlags = 8;
 struct SolveArgs {
     PlanDev plan;
     const double* etot;   // [M][120] per-edge Hii, Hij, Hjj, vi, vj
-    const double* stot;   // [N_pu + N_E][36] Schur pair blocks / row gradients
+    const double* stot;   // [nsp][N_pu + N_E][36] Schur pair blocks / row gradients by pixel share
+    size_t share;         // doubles of stot per share
+    int nsp;
     int N_pu, P, n, n_blk, t0, t1;
     float lm, ep;
     double* S;      // working buffer of the blocked solver (blk_doubles)
@@ -529,6 +671,13 @@ struct SolveArgs {
                         // before the retraction (the overlapped step's ready flag)
 };
 
+// an entry of stot: its pixel shares in order
+__device__ __forceinline__ double stot_sum(const SolveArgs& A, size_t i) {
+    double t = A.stot[i];
+    for (int k = 1; k < A.nsp; k++) t += A.stot[k * A.share + i];
+    return t;
+}
+
 // One edge-block or Schur-item contribution to entry (r, c) of a 6x6 block of
 // S (ba.cuh:520-548, 722-742): code cd of the block's contribution list.
 __device__ __forceinline__ double s_contrib(const SolveArgs& A, int cd, int r, int c) {
@@ -541,7 +690,7 @@ __device__ __forceinline__ double s_contrib(const SolveArgs& A, int cd, int r, i
              : w == 2 ? et[kTotHij + c * 6 + r]
                       : et[kTotHjj + r * 6 + c];
     }
-    return -A.stot[(size_t)v * 36 + (ty == 1 ? r * 6 + c : c * 6 + r)];
+    return -stot_sum(A, (size_t)v * 36 + (ty == 1 ? r * 6 + c : c * 6 + r));
 }
 
 // One workgroup per 6x6 block (a, b) of S (P*P of them) and per 6-entry
@@ -587,7 +736,7 @@ __global__ __launch_bounds__(256) void k_ba_assemble(SolveArgs A) {
                 if (code_type(cd) == 0)
                     s += A.etot[(size_t)(v >> 1) * kNT + ((v & 1) ? kTotVj : kTotVi) + k];
                 else
-                    s -= A.stot[(size_t)(A.N_pu + v) * 36 + k];
+                    s -= stot_sum(A, (size_t)(A.N_pu + v) * 36 + k);
             }
         }
         if (sl < kAsmSlices) red[sl][e] = s;
@@ -1546,7 +1695,7 @@ __global__ __launch_bounds__(256) void k_ba_backsub(PlanDev plan, const double* 
                                                     const double* __restrict__ Wv,
                                                     const float* __restrict__ dx,
                                                     const int* __restrict__ flags,
-                                                    float* __restrict__ disps, int HW) {
+                                                    float* __restrict__ disps, int HW, int HWs) {
     if (flags[0]) return;
     const int kc = blockIdx.y;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1554,12 +1703,12 @@ __global__ __launch_bounds__(256) void k_ba_backsub(PlanDev plan, const double* 
     double dw = 0.0;
     for (int r = plan.kf_rptr[kc]; r < plan.kf_rptr[kc + 1]; r++) {
         const int row = plan.kf_rows[r];
-        const double* er = E + (size_t)row * 6 * HW + k;
+        const double* er = E + (size_t)row * 6 * HWs + k;
         const float* x = dx + plan.row_pose[row] * 6;
 #pragma unroll
-        for (int n = 0; n < 6; n++) dw += er[(size_t)n * HW] * (double)x[n];
+        for (int n = 0; n < 6; n++) dw += er[(size_t)n * HWs] * (double)x[n];
     }
-    const double dz = Q[(size_t)kc * HW + k] * (Wv[(size_t)kc * HW + k] - dw);
+    const double dz = Q[(size_t)kc * HWs + k] * (Wv[(size_t)kc * HWs + k] - dw);
     float* d = disps + (size_t)plan.kf_list[kc] * HW + k;
     *d = (float)((double)*d + dz);
 }
@@ -2571,6 +2720,8 @@ struct BaState {
     int key_t0 = 0, key_t1 = 0, key_motion = 0, key_HW = 0;
     // plan sizes
     int M = 0, P = 0, n = 0, N_kf = 0, N_E = 0, N_pu = 0, n_blk = 0, nch = 1;
+    int n_zitems = 0, nsp = 1;  // k_ba_schur: items, pixel shares
+    int HWs = 0;  // row stride of E, Q, Wv
     int npose = 0;  // max(the edges' largest frame index + 1, t1)
     std::vector<int> host;  // packed plan
     size_t off[kPlanParts] = {0};
@@ -2594,8 +2745,8 @@ PlanDev plan_ptrs(BaState* s) {
     const int* base = s->plan_dev.as<int>();
     PlanDev p;
     const int** f[kPlanParts] = {&p.kf_list, &p.kf_eptr, &p.kf_eidx, &p.edge_ri, &p.edge_rj,
-                                 &p.row_pose, &p.row_kf, &p.kf_rptr, &p.kf_rows, &p.pairs,
-                                 &p.sblk, &p.sblk_ptr, &p.sblk_src, &p.bv_ptr, &p.bv_src,
+                                 &p.row_pose, &p.row_kf, &p.kf_rptr, &p.kf_rows, &p.zitems,
+                                 &p.kf_pbase, &p.sblk, &p.sblk_ptr, &p.sblk_src, &p.bv_ptr, &p.bv_src,
                                  &p.blkmap};
     for (int i = 0; i < kPlanParts; i++) *f[i] = base + s->off[i];
     return p;
@@ -2768,15 +2919,37 @@ int build_plan(BaState* s, const int* ii, const int* jj, int M, int t0, int t1, 
         std::vector<int> fill(kf_rptr.begin(), kf_rptr.end() - 1);
         for (int r = 0; r < N_E; r++) kf_rows[fill[row_kf[r]]++] = r;
     }
-    std::vector<int> pairs;
-    for (int kc = 0; kc < N_kf; kc++)
+    // the keyframes' items of k_ba_schur, those with the most tiles first (the
+    // launch's last workgroups are then short)
+    std::vector<std::array<int, 4>> zi;
+    for (int kc = 0; kc < N_kf; kc++) {
+        const int nr = kf_rptr[kc + 1] - kf_rptr[kc];
+        const int T = nr > 0 ? (6 * nr + 16) / 16 : 0;
+        for (int a = 0; a < T; a += kSchT) {
+            const int d = std::min(kSchT, T - a);
+            zi.push_back({d * (d + 1) / 2, kc, a, a});
+            for (int b = a + kSchT; b < T; b += kSchTB)
+                zi.push_back({kSchT * std::min(kSchTB, T - b), kc, a, b});
+        }
+    }
+    std::stable_sort(zi.begin(), zi.end(),
+                     [](const std::array<int, 4>& x, const std::array<int, 4>& y) {
+                         return x[0] > y[0];
+                     });
+    s->n_zitems = (int)zi.size();
+    std::vector<int> zitems;
+    for (const auto& z : zi) zitems.insert(zitems.end(), {z[1], z[2], z[3]});
+    // upper pairs of a keyframe's rows
+    std::vector<int> pairs, kf_pbase;
+    for (int kc = 0; kc < N_kf; kc++) {
+        kf_pbase.push_back((int)pairs.size() / 2);
         for (int a = kf_rptr[kc]; a < kf_rptr[kc + 1]; a++)
             for (int b = a; b < kf_rptr[kc + 1]; b++) {
                 pairs.push_back(kf_rows[a]);
                 pairs.push_back(kf_rows[b]);
-                pairs.push_back(kc);
             }
-    const int N_pu = (int)pairs.size() / 3;
+    }
+    const int N_pu = (int)pairs.size() / 2;
     // contributions per destination block a*P+b
     std::map<int, std::vector<int>> blocks;
     for (int e = 0; e < M; e++) {
@@ -2790,7 +2963,7 @@ int build_plan(BaState* s, const int* ii, const int* jj, int M, int t0, int t1, 
         if (vb) blocks[b * P + b].push_back(code(0, e * 4 + 3));
     }
     for (int p = 0; p < N_pu; p++) {
-        const int r1 = pairs[3 * p], r2 = pairs[3 * p + 1];
+        const int r1 = pairs[2 * p], r2 = pairs[2 * p + 1];
         const int a = row_pose[r1], b = row_pose[r2];
         blocks[a * P + b].push_back(code(1, p));
         if (r1 != r2) blocks[b * P + a].push_back(code(2, p));
@@ -2822,7 +2995,7 @@ int build_plan(BaState* s, const int* ii, const int* jj, int M, int t0, int t1, 
     for (size_t k = 0; k < sblk.size(); k++) blkmap[sblk[k]] = (int)k;
     const std::vector<int>* parts[kPlanParts] = {&kf_list, &kf_eptr, &kf_eidx, &edge_ri,
                                                  &edge_rj, &row_pose, &row_kf, &kf_rptr,
-                                                 &kf_rows, &pairs, &sblk, &sblk_ptr,
+                                                 &kf_rows, &zitems, &kf_pbase, &sblk, &sblk_ptr,
                                                  &sblk_src, &bv_ptr, &bv_src, &blkmap};
     s->host.clear();
     for (int i = 0; i < kPlanParts; i++) {
@@ -2902,6 +3075,11 @@ int ba_prepare(slk_ctx* ctx, const IterArgs& I, const int* ii_host, const int* j
     s->valid = false;
     SLK_TRY(build_plan(s, ii_host, jj_host, M, t0, t1, motion_only, HW));
     if (s->n > 0x7fff) return fail(SLK_E_ARG, "ba_iterate: too many free poses");
+    // pixel shares of k_ba_schur: about four workgroups a CU, each of its waves
+    // at least two runs of 16 pixels
+    s->HWs = (HW + 15) / 16 * 16;
+    s->nsp = std::max(1, std::min({(4 * s->cus + s->n_zitems - 1) / std::max(1, s->n_zitems),
+                                   s->HWs / 128, 8}));
     const size_t pbytes = s->host.size() * sizeof(int);
     SLK_TRY(s->stage.ensure(pbytes));
     std::memcpy(s->stage.ptr, s->host.data(), pbytes);
@@ -2918,11 +3096,11 @@ int ba_prepare(slk_ctx* ctx, const IterArgs& I, const int* ii_host, const int* j
         SLK_TRY(s->ready.ensure(sizeof(int)));
     } else {
         SLK_TRY(s->etot.ensure((size_t)M * kNT * sizeof(double)));
-        SLK_TRY(s->stot.ensure(std::max<size_t>(1, (size_t)(s->N_pu + s->N_E) * 36) *
+        SLK_TRY(s->stot.ensure(std::max<size_t>(1, (size_t)(s->N_pu + s->N_E) * 36 * s->nsp) *
                                sizeof(double)));
-        SLK_TRY(s->E.ensure(std::max<size_t>(1, (size_t)s->N_E * 6 * HW) * sizeof(double)));
-        SLK_TRY(s->Q.ensure((size_t)s->N_kf * HW * sizeof(double)));
-        SLK_TRY(s->Wv.ensure((size_t)s->N_kf * HW * sizeof(double)));
+        SLK_TRY(s->E.ensure(std::max<size_t>(1, (size_t)s->N_E * 6 * s->HWs) * sizeof(double)));
+        SLK_TRY(s->Q.ensure((size_t)s->N_kf * s->HWs * sizeof(double)));
+        SLK_TRY(s->Wv.ensure((size_t)s->N_kf * s->HWs * sizeof(double)));
     }
     if (n > (size_t)kPanelN) SLK_TRY(s->S.ensure(blk_doubles(s->n) * sizeof(double)));
     SLK_TRY(s->S_dbg.ensure(n * n * sizeof(double)));
@@ -2944,6 +3122,8 @@ SolveArgs solve_args(BaState* s, const PlanDev& plan, const IterArgs& I) {
     A.plan = plan;
     A.etot = s->etot.as<double>();
     A.stot = s->stot.as<double>();
+    A.share = (size_t)(s->N_pu + s->N_E) * 36;
+    A.nsp = s->nsp;
     A.N_pu = s->N_pu;
     A.P = s->P;
     A.n = s->n;
@@ -2994,17 +3174,25 @@ int iterate_classic(slk_ctx* ctx, BaState* s, const IterArgs& I, hipStream_t str
                            dim3(kLinWG), 0, stream, plan, I.target, I.weight, I.poses, I.disps,
                            I.intr, I.ii_gpu, I.jj_gpu, I.eta, s->hpart.as<double>(),
                            s->E.as<double>(), s->Q.as<double>(), s->Wv.as<double>(), HW,
-                           ctx->w, s->nch, I.motion_only);
+                           s->HWs, ctx->w, s->nch, I.motion_only);
     }
     SLK_HIP(hipGetLastError());
     {
-        // the Schur items, then one workgroup per edge for its totals
-        const int items = I.motion_only ? 0 : s->N_pu + s->N_E;
         ProfScope ps(ctx, "ba_schur", stream);
-        hipLaunchKernelGGL(k_ba_schur, dim3(items + M), dim3(kSchWG), 0, stream, plan,
-                           s->E.as<double>(), s->Q.as<double>(), s->Wv.as<double>(),
-                           s->stot.as<double>(), HW, s->N_pu, items, I.poses, I.ii_gpu,
+        hipLaunchKernelGGL(k_ba_etot, dim3(M), dim3(64), 0, stream, I.poses, I.ii_gpu,
                            I.jj_gpu, s->hpart.as<double>(), s->etot.as<double>(), s->nch);
+        SchurArgs Z;
+        Z.plan = plan;
+        Z.E = s->E.as<double>();
+        Z.Q = s->Q.as<double>();
+        Z.Wv = s->Wv.as<double>();
+        Z.stot = s->stot.as<double>();
+        Z.HWs = s->HWs;
+        Z.N_pu = s->N_pu;
+        Z.nsp = s->nsp;
+        Z.share = (size_t)(s->N_pu + s->N_E) * 36;
+        if (s->n_zitems > 0)
+            hipLaunchKernelGGL(k_ba_schur, dim3(s->n_zitems * s->nsp), dim3(256), 0, stream, Z);
         SLK_HIP(hipGetLastError());
     }
     const SolveArgs A = solve_args(s, plan, I);
@@ -3018,7 +3206,8 @@ int iterate_classic(slk_ctx* ctx, BaState* s, const IterArgs& I, hipStream_t str
         ProfScope ps(ctx, "ba_backsub", stream);
         hipLaunchKernelGGL(k_ba_backsub, dim3((HW + 255) / 256, s->N_kf), dim3(256), 0, stream,
                            plan, s->E.as<double>(), s->Q.as<double>(), s->Wv.as<double>(),
-                           s->dx.as<float>(), s->flags.as<int>(), I.disps, HW);
+                           s->dx.as<float>(), s->flags.as<int>(), I.disps, HW,
+                           s->HWs);
         SLK_HIP(hipGetLastError());
     }
     return SLK_OK;

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from helpers import announce, gpu_or_fail, norm_rel
+from oracle import oracle as orc
 import workloads as wl
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +59,34 @@ def test_failed_pivot_in_a_later_block(slk, frame):
     np.testing.assert_array_equal(d["poses"].to_host(), p["poses"])
     np.testing.assert_array_equal(d["disps"].to_host(), p["disps"])
     ctx.close()
+
+
+@pytest.mark.parametrize("h,w,hub", [(7, 9, 9), (7, 9, 14), (37, 53, 16), (7, 9, 40)])
+def test_schur_products_of_many_rows(slk, h, w, hub):
+    """A keyframe with `hub` E rows (frame 1 is fixed) beside keyframes with few: 4, 6, 7 and
+    16 row tiles of k_ba_schur (one group, a second one of a single tile, of
+    two, and several), on maps whose pixels are no multiple of 16, one of
+    them large enough for several pixel shares. S and b against the oracle:
+    both are fp64 sums of h*w products of a few rounded factors each, so they
+    agree to about 4 h w eps of their norm."""
+    orc.build()
+    announce(f"ba schur {h}x{w} hub {hub}")
+    n = hub + 4
+    ii, jj = wl.cyclic_edges(n)
+    extra = [j for j in range(2, n) if j != 3 and (3, j) not in set(zip(ii.tolist(), jj.tolist()))]
+    need = hub - 4
+    ii = np.concatenate([ii, np.full(need, 3, np.int32)])
+    jj = np.concatenate([jj, np.asarray(extra[:need], np.int32)])
+    p = wl.ba_problem(n=n, h=h, w=w, ii=ii, jj=jj, seed=50 + hub)
+    ctx, d = _run(slk, p, 1e-4, 0.1)
+    assert ctx.ba_status() == slk.SLK_OK
+    S, b, _ = ctx.ba_last_system()
+    ctx.close()
+    ref = orc.ba_iterate(p["poses"], p["disps"], p["intr"], p["target"], p["weight"], p["eta"],
+                         p["ii"], p["jj"], h, w, p["t0"], p["t1"], 1e-4, 0.1)
+    bound = 4 * h * w * np.finfo(float).eps
+    print(f"S {norm_rel(S, ref['S']):.2e} b {norm_rel(b, ref['b']):.2e} bound {bound:.1e}")
+    assert norm_rel(S, ref["S"]) < bound
+    assert norm_rel(b, ref["b"]) < bound
+    assert norm_rel(d["poses"].to_host(), ref["poses"]) < 1e-6
+    assert norm_rel(d["disps"].to_host().reshape(-1), ref["disps"].reshape(-1)) < 1e-6
