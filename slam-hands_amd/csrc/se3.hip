@@ -79,10 +79,17 @@ __global__ void k_disp_retr(float* __restrict__ disps, const float* __restrict__
 }
 
 // Mean flow magnitude of the full and the translation-only reprojection
-// (se3.cuh:209-277), one wavefront per pair (four pairs per workgroup): every
-// lane forms the pair's relative pose itself (uniform arithmetic, no barrier),
-// takes pixels lane, lane + 64, ... and the three sums are reduced across the
+// (se3.cuh:209-277), one wavefront per pair (four pairs per workgroup). The
+// relative pose is formed once per pair, in double, as the matrix that takes
+// a pixel's offset (u - cx, v - cy, 1, disparity) to fx X, fy Y and Z, each
+// coefficient rounded once: a pixel is then 12 FMAs and two reciprocals and
+// square roots (v_rcp_f32, v_sqrt_f32, 1 ulp; the reference builds with
+// --use_fast_math). Lane l takes pixels l, l + 64, ..., four loads in flight;
+// valid pixels are counted by ballot, and the sums are reduced across the
 // wavefront in a fixed order (deterministic).
+// What bounds it: vector issue, about 50 instructions a pixel. 40,000 pairs
+// of 48x64: 298 us with the quaternion applied per pixel (an integer division
+// and ~110 instructions), 138 us so.
 __global__ __launch_bounds__(256) void k_frame_distance(const float* __restrict__ poses,
                                                         const float* __restrict__ disps,
                                                         const float* __restrict__ intr,
@@ -93,59 +100,92 @@ __global__ __launch_bounds__(256) void k_frame_distance(const float* __restrict_
     const int e = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     if (e >= M) return;  // uniform over the wavefront
     const int lane = threadIdx.x & 63;
-    float tij[3], qij[4];
-    {
-        float ti[3], qi[4], tj[3], qj[4];
-        load_pose(poses, ii[e], ti, qi);
-        load_pose(poses, jj[e], tj, qj);
-        rel_se3(ti, qi, tj, qj, tij, qij);
-    }
-    const float fx = intr[0], fy = intr[1], cx = intr[2], cy = intr[3];
-    // the reference builds with --use_fast_math (approximate divisions); here
-    // each projection takes one hardware reciprocal (v_rcp_f32, 1 ulp) of the
-    // depth and the normalised coordinates one reciprocal of each focal length
-    const float ifx = 1.0f / fx, ify = 1.0f / fy;
-    const int HW = H * W;
     const int ix = ii[e];
-    float acc[3] = {0.0f, 0.0f, 0.0f};  // accum, valid, total
-    for (int k = lane; k < HW; k += 64) {
-        const int i = k / W, j = k - (k / W) * W;
-        const float u = (float)j, v = (float)i;
-        float Xi[4], Xj[4];
-        Xi[0] = (u - cx) * ifx;
-        Xi[1] = (v - cy) * ify;
-        Xi[2] = 1.0f;
-        Xi[3] = disps[(size_t)ix * HW + k];
-        act_se3(tij, qij, Xi, Xj);
-        float iz = __builtin_amdgcn_rcpf(Xj[2]);
-        float du = fx * (Xj[0] * iz) + cx - u, dv = fy * (Xj[1] * iz) + cy - v;
-        float d = sqrtf(du * du + dv * dv);
-        acc[2] += beta;
-        if (Xj[2] > kMinDepth) {
-            acc[0] += beta * d;
-            acc[1] += beta;
+    const float cx = intr[2], cy = intr[3];
+    // rows fx X, fy Y, Z of the map; t: its disparity column
+    float a[3][3], t[3];
+    {
+        const double fx = intr[0], fy = intr[1];
+        double ti[3], qi[4], tj[3], qj[4], tij[3], q[4];
+        load_pose(poses, ix, ti, qi);
+        load_pose(poses, jj[e], tj, qj);
+        rel_se3(ti, qi, tj, qj, tij, q);
+        const double f[3] = {fx, fy, 1.0};
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const double X[3] = {c == 0 ? 1.0 : 0.0, c == 1 ? 1.0 : 0.0, c == 2 ? 1.0 : 0.0};
+            double Y[3];
+            act_so3(q, X, Y);  // column c of the rotation
+#pragma unroll
+            for (int r = 0; r < 3; r++) a[r][c] = (float)(f[r] * Y[r] / f[c]);
         }
-        Xj[0] = Xi[0] + Xi[3] * tij[0];
-        Xj[1] = Xi[1] + Xi[3] * tij[1];
-        Xj[2] = Xi[2] + Xi[3] * tij[2];
-        iz = __builtin_amdgcn_rcpf(Xj[2]);
-        du = fx * (Xj[0] * iz) + cx - u;
-        dv = fy * (Xj[1] * iz) + cy - v;
-        d = sqrtf(du * du + dv * dv);
-        acc[2] += (1.0f - beta);
-        if (Xj[2] > kMinDepth) {
-            acc[0] += (1.0f - beta) * d;
-            acc[1] += (1.0f - beta);
+#pragma unroll
+        for (int r = 0; r < 3; r++) t[r] = (float)(f[r] * tij[r]);
+    }
+    const int HW = H * W;
+    const float* dp = disps + (size_t)ix * HW;
+    float s1 = 0.0f, s2 = 0.0f;
+    int n1 = 0, n2 = 0;
+    auto pixel = [&](float u, float v, float d, bool in) {
+        const float x = u - cx, y = v - cy;
+        float X = fmaf(a[0][0], x, fmaf(a[0][1], y, fmaf(t[0], d, a[0][2])));
+        float Y = fmaf(a[1][0], x, fmaf(a[1][1], y, fmaf(t[1], d, a[1][2])));
+        float Z = fmaf(a[2][0], x, fmaf(a[2][1], y, fmaf(t[2], d, a[2][2])));
+        float iz = __builtin_amdgcn_rcpf(Z);
+        float du = fmaf(X, iz, -x), dv = fmaf(Y, iz, -y);
+        bool ok = in && Z > kMinDepth;
+        s1 += ok ? __builtin_amdgcn_sqrtf(fmaf(du, du, dv * dv)) : 0.0f;
+        n1 += __popcll(__ballot(ok));
+        X = fmaf(t[0], d, x);
+        Y = fmaf(t[1], d, y);
+        Z = fmaf(t[2], d, 1.0f);
+        iz = __builtin_amdgcn_rcpf(Z);
+        du = fmaf(X, iz, -x);
+        dv = fmaf(Y, iz, -y);
+        ok = in && Z > kMinDepth;
+        s2 += ok ? __builtin_amdgcn_sqrtf(fmaf(du, du, dv * dv)) : 0.0f;
+        n2 += __popcll(__ballot(ok));
+    };
+    // (u, v) of pixel k, stepped by 64 pixels at a time (whole numbers: exact)
+    const int v0 = lane / W;
+    float u = (float)(lane - v0 * W), v = (float)v0;
+    const float du64 = (float)(64 % W), dv64 = (float)(64 / W), fw = (float)W;
+    auto step = [&]() {
+        u += du64;
+        v += dv64;
+        const bool wrap = u >= fw;
+        u = wrap ? u - fw : u;
+        v = wrap ? v + 1.0f : v;
+    };
+    int k = lane;
+    for (; k - lane + 256 <= HW; k += 256) {
+        float d[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) d[q] = dp[k + 64 * q];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            pixel(u, v, d[q], true);
+            step();
         }
     }
+    for (; k - lane < HW; k += 64) {
+        pixel(u, v, dp[min(k, HW - 1)], k < HW);
+        step();
+    }
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1)
-#pragma unroll
-        for (int q = 0; q < 3; q++) acc[q] += __shfl_xor(acc[q], off, 64);
-    if (lane == 0)
-        dist[e] = (acc[1] / (acc[2] + 1e-8f) < 0.75f) ? 1000.0f : acc[0] / acc[1];
+    for (int off = 32; off >= 1; off >>= 1) {
+        s1 += __shfl_xor(s1, off, 64);
+        s2 += __shfl_xor(s2, off, 64);
+    }
+    if (lane == 0) {
+        // beta of every valid pixel of the one, 1 - beta of the other: whole
+        // multiples, rounded to fp32 once
+        const double b = beta;
+        const float val = (float)(b * n1 + (1.0 - b) * n2), all = (float)HW;
+        const float sum = fmaf(beta, s1, (1.0f - beta) * s2);
+        dist[e] = (val / (all + 1e-8f) < 0.75f) ? 1000.0f : sum / val;
+    }
 }
-
 
 __global__ void k_clamp(float* __restrict__ d, int n, float lo) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;

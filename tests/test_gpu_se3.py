@@ -120,3 +120,22 @@ def test_frame_distance_known_answers(slk, case):
     assert got == pytest.approx(want, rel=1e-5)
     assert got == pytest.approx(float(orc.frame_distance(poses, disps, intr, [0], [1], H, W,
                                                          0.3)[0]), rel=1e-5)
+
+
+@pytest.mark.parametrize("h,w", [(1, 1), (5, 7), (8, 8), (3, 100), (16, 17), (130, 2), (37, 53)])
+def test_frame_distance_map_sizes(slk, h, w):
+    """Maps below one wavefront's 64 pixels, at and past 64 and 256, narrower
+    and wider than 64 columns: fp32 sums of h*w flow magnitudes whose terms
+    are good to a few ulp of the image coordinates they are differences of
+    (under 130, so 1e-5 px each)."""
+    announce(f"frame_distance {h}x{w}")
+    pin = Pins(slk)
+    p = wl.ba_problem(n=5, h=h, w=w, ii=np.array([0], np.int32), jj=np.array([1], np.int32), seed=6)
+    ii, jj = (v.reshape(-1).astype(np.int32) for v in np.meshgrid(range(5), range(5), indexing="ij"))
+    d = {k: slk.DeviceArray.from_host(p[k]) for k in ("poses", "disps", "intr")}
+    dist = slk.DeviceArray((25,))
+    slk.check(slk.lib().slk_frame_distance(d["poses"].ptr, d["disps"].ptr, d["intr"].ptr, pin(ii),
+                                           pin(jj), dist.ptr, 25, h, w, 0.3, None))
+    slk.hip().sync()
+    ref = orc.frame_distance(p["poses"], p["disps"], p["intr"], ii, jj, h, w, 0.3)
+    np.testing.assert_allclose(dist.to_host(), ref, rtol=1e-5, atol=1e-4)
