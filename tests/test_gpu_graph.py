@@ -80,6 +80,20 @@ def test_proximity_factors(slk, case):
     assert np.sum(dist[(pi - pj) > rad + 1] <= thresh) > 0  # the greedy step had candidates
 
 
+MORE_CASES = [  # no suppression; one that closes nothing; t1 past t0; limits at both ends
+    ("no_nms", 0, 0, 2, -1, 16.0, 30, 10, 0),
+    ("thresh_past_closed", 0, 0, 1, 2, 2e6, 30, 10, 0),
+    ("thresh_past_100", 0, 0, 1, 3, 500.0, 30, 10, 90),
+    ("t1_past_t0", 4, 9, 1, 2, 16.0, 30, 10, 0),
+    ("no_radius", 0, 0, -1, 4, 16.0, 60, 0, 70),
+]
+
+
+@pytest.mark.parametrize("case", MORE_CASES, ids=[c[0] for c in MORE_CASES])
+def test_proximity_factors_odd_parameters(slk, case):
+    test_proximity_factors(slk, case)
+
+
 # ------------------------------------------- edge-state update (main.cu:795-836)
 EDGE_CASES = [  # (name, n, removed, inactive already held, max_inac)
     ("age_removal", 48, [3, 17, 18, 40], 5, 64),
