@@ -606,7 +606,7 @@ __device__ __forceinline__ void window_to_channels(const float (&win)[8][8], flo
 // One thread per (source pixel, level, edge): zero-padded bilinear samples at
 // (x0 - 3 + a, y0 - 3 + b), a,b in [0,7), from that pixel's own row of the
 // level (main.cu:1175-1217). Non-finite coordinates give zeros.
-__global__ __launch_bounds__(256) void k_corr_lookup(LevelIn lv, const float* __restrict__ coords,
+__global__ __launch_bounds__(64) void k_corr_lookup(LevelIn lv, const float* __restrict__ coords,
                                                      float* __restrict__ out, int HW1,
                                                      int level_base, int nch) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -627,18 +627,22 @@ __global__ __launch_bounds__(256) void k_corr_lookup(LevelIn lv, const float* __
     }
     const int ix = win_origin(cx, lvl), iy = win_origin(cy, lvl);
     const float* vol = lv.p[l] + ((size_t)e * HW1 + p) * (size_t)(H2 * W2);
+    // all 64 loads unconditional, from the nearest cell of the level, and
+    // masked after (a load under its own test waits before the next one: 29 us
+    // for the 4 levels of a 48x64 map, 5.4 us so)
     float win[8][8];
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        const int y = iy + j;
-        const bool vy = (unsigned)y < (unsigned)H2;
+        const int y = min(max(iy + j, 0), H2 - 1);
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int x = ix + i;
-            const bool ok = vy && (unsigned)x < (unsigned)W2;
-            win[j][i] = ok ? vol[y * W2 + x] : 0.0f;
-        }
+        for (int i = 0; i < 8; i++) win[j][i] = vol[y * W2 + min(max(ix + i, 0), W2 - 1)];
     }
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if ((unsigned)(iy + j) >= (unsigned)H2 || (unsigned)(ix + i) >= (unsigned)W2)
+                win[j][i] = 0.0f;
     window_to_channels(win, x0 - floorf(x0), y0 - floorf(y0), o, HW1);
 }
 
@@ -731,9 +735,10 @@ int launch_tile(slk_ctx* ctx, const Tin* fa, const Tin* fb, long fstride, const 
 int launch_lookup(slk_ctx* ctx, const LevelIn& lv, int nlev, int level_base, int nch,
                   const float* coords, float* out, int B, int HW1, hipStream_t stream) {
     if (B <= 0) return SLK_OK;
-    dim3 grid((HW1 + 255) / 256, nlev, B);
+    // one wave a workgroup: a single edge's 48x64 map then covers 192 CUs
+    dim3 grid((HW1 + 63) / 64, nlev, B);
     ProfScope ps(ctx, "corr_lookup", stream);
-    hipLaunchKernelGGL(k_corr_lookup, grid, dim3(256), 0, stream, lv, coords, out, HW1, level_base,
+    hipLaunchKernelGGL(k_corr_lookup, grid, dim3(64), 0, stream, lv, coords, out, HW1, level_base,
                        nch);
     SLK_HIP(hipGetLastError());
     return SLK_OK;
