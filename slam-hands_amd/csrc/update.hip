@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "lds_dma.hpp"
+#include "reduce.hpp"
 #include "slk_internal.hpp"
 
 namespace slk {
@@ -47,7 +48,42 @@ constexpr int kTW = 32;   // output columns per workgroup tile (one MFMA column 
 constexpr int kCoT = 128; // output channels per workgroup tile
 
 __device__ __forceinline__ float r16(float x) { return (float)(_Float16)x; }
-__device__ __forceinline__ float sigm(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// The epilogues' sigmoid and tanh. The library's expf, tanhf and IEEE division
+// took most of them: 10 us of a convz|convr workgroup's 49 and 18 us of a
+// convq one's 64 (per value about 240 and 440 cycles of its wave). These are
+// straight-line fp32, within 3 ulp, from v_exp_f32 and v_rcp_f32 (1 ulp each);
+// every result is rounded to fp16 next. NaN stays NaN.
+//
+// e^x = 2^(x log2 e): the product's rounding error and log2 e's own go back in
+// through the first-order factor; |x| large is clamped where the results of
+// sigm and tanh_f32 no longer depend on it.
+__device__ __forceinline__ float exp_f32(float x) {
+    x = x > 88.0f ? 88.0f : x < -104.0f ? -104.0f : x;
+    const float t = x * 1.44269502f;
+    const float r = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e, r * 0.693147182f, e);
+}
+// 1/d for 1 <= d < 2^127: estimate and one Newton step
+__device__ __forceinline__ float rcp_f32(float d) {
+    const float y = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float sigm(float x) { return rcp_f32(1.0f + exp_f32(-x)); }
+// tanh: the Taylor series to x^13 below 0.4 (its next term is 4e-9 of the
+// sum there), 1 - 2 / (e^(2|x|) + 1) above
+__device__ __forceinline__ float tanh_f32(float x) {
+    const float a = fabsf(x), q = x * x;
+    float p = fmaf(q, 3.59212804e-3f, -8.86323552e-3f);
+    p = fmaf(q, p, 2.18694885e-2f);
+    p = fmaf(q, p, -5.39682540e-2f);
+    p = fmaf(q, p, 1.33333333e-1f);
+    p = fmaf(q, p, -3.33333333e-1f);
+    p = fmaf(x * q, p, x);
+    const float z = fmaf(-2.0f, rcp_f32(exp_f32(2.0f * a) + 1.0f), 1.0f);
+    return a < 0.4f ? p : copysignf(z, x);
+}
 
 // One input source of a convolution: chunks of a CK buffer.
 struct CkSrc {
@@ -62,6 +98,7 @@ enum Epi {
     kEpiZR = 2,     // rows < 128: z; rows >= 128: r and out r*net (see below)
     kEpiQ = 3,      // q and the state update
     kEpiHeads = 4,  // rows < 256: out16 = round16(relu(conv + b)); rows >= 256: out32
+    kEpiPart = 5,   // the sums of a share of the input chunks, for k_conv_reduce
 };
 
 struct ConvArgs {
@@ -82,119 +119,242 @@ struct ConvArgs {
     const float* gterm;   // [image][384] rounded global terms (zg | rg | qg)
     float* out32;         // kEpiQ: the new state; kEpiHeads: agg_conv1, NCHW fp32
     long out32_nstride;
+    // chunks split over nsplit workgroups (k_conv3): sums of a share,
+    // [image * nsplit + share][co_tot / 4][hw][4]
+    float* part;
+    int nsplit;
     const _Float16* zero16;  // 16 zero bytes: the source of staged units outside the image
 };
 
-// The epilogue of one pixel's two 32-row accumulator blocks: acc0/acc1
-// register v holds output channel co0 + mb*32 + 8*(v/4) + v%4 (co0 includes
-// the lane's 4*lhi), so each group of four registers is four consecutive
-// channels of the CK layout. bias[co] is the channel's bias and, for kEpiZR
-// and kEpiQ, gts[co] its global term of image n (the 3x3 kernels stage
-// their tile's in LDS). Every memory read of the epilogue is
-// issued before its first store, from a clamped channel where the group is
-// past Co: vector memory counts loads and stores together, in order, so a
-// load issued after a store would wait for that store.
+// Image n's part of an epilogue buffer, and an element of it by a 32-bit byte
+// offset (an image's channels stay under 2^31 bytes at the largest map,
+// h w = 2^22), so an access is a scalar base plus one offset register.
+template <typename T, typename E>
+__device__ __forceinline__ T& epi_at(E* base, unsigned elem) {
+    return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + elem * (unsigned)sizeof(E));
+}
+template <typename T, typename E>
+__device__ __forceinline__ const T& epi_at(const E* base, unsigned elem) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) +
+                                       elem * (unsigned)sizeof(E));
+}
+// element of channel co of pixel p in a CK image
+__device__ __forceinline__ unsigned ck_elem(int co, int p, int HW) {
+    return ((unsigned)(co >> 4) * HW + p) * 16 + (co & 15);
+}
+
+// The arguments with every epilogue buffer at image n (of part: n counts
+// image and share)
+__device__ __forceinline__ ConvArgs epi_image(ConvArgs a, int n, int HW) {
+    a.out16 += (long)n * a.out16_nstride;
+    a.zbuf += (long)n * a.zr_nstride;
+    a.rnet += (long)n * a.zr_nstride;
+    a.net16 += (long)n * a.net_nstride;
+    a.out32 += (long)n * a.out32_nstride;
+    a.part += (long)n * a.co_tot * HW;
+    return a;
+}
+
+// The stores of four consecutive output channels co .. co + 3 of pixel p of
+// the image: v is the convolution with its bias, gts the channels' global terms
+// (kEpiZR, kEpiQ), s0 and s1 the state operands epi_read loaded.
 template <int EPI>
-__device__ __forceinline__ void epi_block(const ConvArgs& a, const f32x16& acc0,
-                                          const f32x16& acc1, int n, int co0, int p, int HW,
-                                          const float* bias, const float* gts) {
-    // the state operands of each group: s0 (net, or for kEpiQ z), s1 (kEpiQ: net)
-    f16x4 s0[2][4], s1[2][4];
+__device__ __forceinline__ void epi_store(const ConvArgs& a, const float (&v)[4], const float* gts,
+                                          const f16x4& s0, const f16x4& s1, int co, int p,
+                                          int HW) {
+    if constexpr (EPI == kEpiRelu) {
+        f16x4 o;
 #pragma unroll
-    for (int mb = 0; mb < 2; mb++)
+        for (int i = 0; i < 4; i++) o[i] = (_Float16)fmaxf(v[i], 0.0f);
+        epi_at<f16x4>(a.out16, ck_elem(co, p, HW)) = o;
+    } else if constexpr (EPI == kEpiGate) {
+        f16x4 o;
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int co = co0 + mb * 32 + 8 * g;
-            const int cc = co < a.Co ? co : 0;
-            if constexpr (EPI == kEpiGate) {
-                s0[mb][g] = *reinterpret_cast<const f16x4*>(
-                    a.net16 + (long)n * a.net_nstride + ((long)(cc >> 4) * HW + p) * 16 + (cc & 15));
-            } else if constexpr (EPI == kEpiZR) {
-                const int cr = cc >= 128 ? cc - 128 : 0;
-                s0[mb][g] = *reinterpret_cast<const f16x4*>(
-                    a.net16 + (long)n * a.net_nstride + ((long)(cr >> 4) * HW + p) * 16 + (cr & 15));
-            } else if constexpr (EPI == kEpiQ) {
-                const long off = ((long)(cc >> 4) * HW + p) * 16 + (cc & 15);
-                s0[mb][g] = *reinterpret_cast<const f16x4*>(a.zbuf + (long)n * a.zr_nstride + off);
-                s1[mb][g] = *reinterpret_cast<const f16x4*>(a.net16 + (long)n * a.net_nstride + off);
-            }
+        for (int i = 0; i < 4; i++) o[i] = (_Float16)(r16(sigm(r16(v[i]))) * (float)s0[i]);
+        epi_at<f16x4>(a.out16, ck_elem(co, p, HW)) = o;
+    } else if constexpr (EPI == kEpiZR) {
+        f16x4 sg;
+#pragma unroll
+        for (int i = 0; i < 4; i++) sg[i] = (_Float16)sigm(r16(v[i]) + gts[i]);
+        if (co < 128) {  // uniform
+            epi_at<f16x4>(a.zbuf, ck_elem(co, p, HW)) = sg;
+        } else {
+            f16x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[i] = (_Float16)((float)s0[i] * (float)sg[i]);
+            epi_at<f16x4>(a.rnet, ck_elem(co - 128, p, HW)) = o;
         }
+    } else if constexpr (EPI == kEpiQ) {
+        f16x4 o;
+        float* out32 = a.out32;
 #pragma unroll
-    for (int mb = 0; mb < 2; mb++) {
-        const f32x16& acc = mb ? acc1 : acc0;
+        for (int i = 0; i < 4; i++) {
+            const float q = r16(tanh_f32(r16(v[i]) + gts[i]));
+            const float zi = (float)s0[i];
+            const float nn = (1.0f - zi) * (float)s1[i] + zi * q;
+            o[i] = (_Float16)nn;
+            epi_at<float>(out32, (unsigned)(co + i) * HW + p) = (float)o[i];
+        }
+        epi_at<f16x4>(a.net16, ck_elem(co, p, HW)) = o;
+    } else {  // kEpiHeads
+        if (co < 256) {  // uniform
+            f16x4 o;
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int co = co0 + mb * 32 + 8 * g;
-            if (co >= a.Co) continue;
-            float v[4];
+            for (int i = 0; i < 4; i++) o[i] = (_Float16)fmaxf(v[i], 0.0f);
+            epi_at<f16x4>(a.out16, ck_elem(co, p, HW)) = o;
+        } else {
+            float* out32 = a.out32;
 #pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = acc[4 * g + i] + bias[co + i];
-            if constexpr (EPI == kEpiRelu) {
-                f16x4 o;
-#pragma unroll
-                for (int i = 0; i < 4; i++) o[i] = (_Float16)fmaxf(v[i], 0.0f);
-                *reinterpret_cast<f16x4*>(a.out16 + (long)n * a.out16_nstride +
-                                          ((long)(co >> 4) * HW + p) * 16 + (co & 15)) = o;
-            } else if constexpr (EPI == kEpiGate) {
-                const f16x4 nt = s0[mb][g];
-                f16x4 o;
-#pragma unroll
-                for (int i = 0; i < 4; i++) o[i] = (_Float16)(r16(sigm(r16(v[i]))) * (float)nt[i]);
-                *reinterpret_cast<f16x4*>(a.out16 + (long)n * a.out16_nstride +
-                                          ((long)(co >> 4) * HW + p) * 16 + (co & 15)) = o;
-            } else if constexpr (EPI == kEpiZR) {
-                f16x4 sg;
-#pragma unroll
-                for (int i = 0; i < 4; i++) sg[i] = (_Float16)sigm(r16(v[i]) + gts[co + i]);
-                if (co < 128) {
-                    *reinterpret_cast<f16x4*>(a.zbuf + (long)n * a.zr_nstride +
-                                              ((long)(co >> 4) * HW + p) * 16 + (co & 15)) = sg;
-                } else {
-                    const int cr = co - 128;
-                    const long off = ((long)(cr >> 4) * HW + p) * 16 + (cr & 15);
-                    const f16x4 nt = s0[mb][g];
-                    f16x4 o;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) o[i] = (_Float16)((float)nt[i] * (float)sg[i]);
-                    *reinterpret_cast<f16x4*>(a.rnet + (long)n * a.zr_nstride + off) = o;
-                }
-            } else if constexpr (EPI == kEpiQ) {
-                const long off = ((long)(co >> 4) * HW + p) * 16 + (co & 15);
-                const f16x4 z = s0[mb][g], nt = s1[mb][g];
-                f16x4 o;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float q = r16(tanhf(r16(v[i]) + gts[co + i]));
-                    const float zi = (float)z[i];
-                    const float nn = (1.0f - zi) * (float)nt[i] + zi * q;
-                    o[i] = (_Float16)nn;
-                    a.out32[(long)n * a.out32_nstride + (long)(co + i) * HW + p] = (float)o[i];
-                }
-                *reinterpret_cast<f16x4*>(a.net16 + (long)n * a.net_nstride + off) = o;
-            } else {  // kEpiHeads
-                if (co < 256) {
-                    f16x4 o;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) o[i] = (_Float16)fmaxf(v[i], 0.0f);
-                    *reinterpret_cast<f16x4*>(a.out16 + (long)n * a.out16_nstride +
-                                              ((long)(co >> 4) * HW + p) * 16 + (co & 15)) = o;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        a.out32[(long)n * a.out32_nstride + (long)(co - 256 + i) * HW + p] =
-                            r16(fmaxf(v[i], 0.0f));
-                }
-            }
+            for (int i = 0; i < 4; i++)
+                epi_at<float>(out32, (unsigned)(co - 256 + i) * HW + p) = r16(fmaxf(v[i], 0.0f));
         }
     }
 }
 
-// 1x1 convolutions as a plain GEMM with register-direct operands (no halo,
-// so nothing is staged in LDS): tile kCoT output channels x 256 consecutive
-// pixels, wave (wm, wn) = 64 channels x 128 pixels; every lane loads its
-// 16-byte A (weights) and B (8 channels of one pixel) fragments straight from
-// global memory, two chunks ahead of their MFMAs.
+// The state operands of channels co .. co + 3: s0 = net (kEpiGate, kEpiZR; its
+// z rows have none and read channel 0's) or z (kEpiQ), s1 = net (kEpiQ).
 template <int EPI>
+__device__ __forceinline__ void epi_read(const ConvArgs& a, int co, int p, int HW, f16x4& s0,
+                                         f16x4& s1) {
+    if constexpr (EPI == kEpiGate)
+        s0 = epi_at<f16x4>(a.net16, ck_elem(co, p, HW));
+    else if constexpr (EPI == kEpiZR)
+        s0 = epi_at<f16x4>(a.net16,
+                           ck_elem(co >= 128 ? co - 128 : 0, p, HW));
+    else if constexpr (EPI == kEpiQ) {
+        s0 = epi_at<f16x4>(a.zbuf, ck_elem(co, p, HW));
+        s1 = epi_at<f16x4>(a.net16, ck_elem(co, p, HW));
+    }
+}
+
+// The epilogue of a wave's MB x R accumulator blocks: block (mb, r) holds 32
+// output channels of 32 pixels, its register v channel co0 + mb*32 + 8*(v/4)
+// + v%4 (co0 includes the lane's 4*lhi), so each group of four registers is
+// four consecutive channels of the CK layout; the lane's pixel of block row r
+// is p[r], stored if in[r] (p[r] is a pixel of the image either way). bias[co]
+// is the channel's bias and, for kEpiZR and kEpiQ, gts[co] its global term of
+// image n (the 3x3 kernels stage their tile's in LDS). Every state operand is
+// read before the first store: vector memory counts loads and stores
+// together, in order, so a load issued after a store would wait for that
+// store. (Row by row, each row's reads behind the row's before it stores, the
+// epilogue took 10 us of a convz|convr workgroup's 49 and 18 us of a convq
+// one's 64.) kEpiPart stores the sums alone, for k_conv_reduce.
+template <int EPI, int MB, int R>
+__device__ __forceinline__ void epi_tile(const ConvArgs& args, const f32x16 (&acc)[MB][R], int n,
+                                         int co0, const int (&p)[R], const bool (&in)[R], int HW,
+                                         const float* bias, const float* gts) {
+    const ConvArgs a = epi_image(args, n, HW);
+    f16x4 s0[R][MB][4], s1[R][MB][4];
+    if constexpr (EPI == kEpiGate || EPI == kEpiZR || EPI == kEpiQ) {
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    epi_read<EPI>(a, co0 + mb * 32 + 8 * g, p[r], HW, s0[r][mb][g], s1[r][mb][g]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (!in[r]) continue;
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int co = co0 + mb * 32 + 8 * g;
+                // only a layer whose channels end inside a tile (Co = 64, a
+                // multiple of the 8 channels of a group's two lane halves) has
+                // rows to leave out: a uniform test
+                if constexpr (EPI == kEpiRelu)
+                    if (__builtin_amdgcn_readfirstlane(co) >= a.Co) continue;
+                if constexpr (EPI == kEpiPart) {
+                    epi_at<float4>(a.part,
+                                   ((unsigned)(co >> 2) * HW + p[r]) * 4) =
+                        float4{acc[mb][r][4 * g], acc[mb][r][4 * g + 1], acc[mb][r][4 * g + 2],
+                               acc[mb][r][4 * g + 3]};
+                } else {
+                    float v[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) v[i] = acc[mb][r][4 * g + i] + bias[co + i];
+                    epi_store<EPI>(a, v, gts + co, s0[r][mb][g], s1[r][mb][g], co, p[r], HW);
+                }
+            }
+    }
+}
+
+// epi_tile of image rows y0 .. y0 + R - 1 at column x
+template <int EPI, int MB, int R>
+__device__ __forceinline__ void epi_rows(const ConvArgs& a, const f32x16 (&acc)[MB][R], int n,
+                                         int co0, int y0, int x, int HW, const float* bias,
+                                         const float* gts) {
+    int p[R];
+    bool in[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        p[r] = min(y0 + r, a.h - 1) * a.w + min(x, a.w - 1);
+        in[r] = y0 + r < a.h && x < a.w;
+    }
+    epi_tile<EPI, MB, R>(a, acc, n, co0, p, in, HW, bias, gts);
+}
+
+// The end of a convolution whose input chunks were split over nsplit
+// workgroups: the shares' sums (part, share k of image n at image index
+// n * nsplit + k) in order, then the epilogue. One thread per pixel and 16
+// channels.
+template <int EPI>
+__global__ __launch_bounds__(64) void k_conv_reduce(ConvArgs args) {
+    const ConvArgs& a = args;
+    const int HW = a.h * a.w, p = blockIdx.x * 64 + threadIdx.x;
+    const int co0 = blockIdx.y * 16, n = blockIdx.z;
+    if (p >= HW) return;
+    const ConvArgs im = epi_image(args, n, HW);
+    f16x4 s0[4], s1[4];
+    float4 sum[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        epi_read<EPI>(im, co0 + 4 * g, p, HW, s0[g], s1[g]);
+        sum[g] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const long stride = (long)(a.co_tot >> 2) * HW * 4;  // floats of a share
+    const float* part = a.part + (long)n * a.nsplit * stride + ((long)(co0 >> 2) * HW + p) * 4;
+    for (int k0 = 0; k0 < a.nsplit; k0 += 4) {  // four shares' loads in flight
+        float4 v[4][4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                v[k][g] = *reinterpret_cast<const float4*>(
+                    part + min(k0 + k, a.nsplit - 1) * stride + (long)g * HW * 4);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (k0 + k < a.nsplit)  // uniform
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    sum[g].x += v[k][g].x;
+                    sum[g].y += v[k][g].y;
+                    sum[g].z += v[k][g].z;
+                    sum[g].w += v[k][g].w;
+                }
+    }
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const int co = co0 + 4 * g;
+        const float* b = a.bias + co;
+        const float v[4] = {sum[g].x + b[0], sum[g].y + b[1], sum[g].z + b[2], sum[g].w + b[3]};
+        const float* gt = a.gterm + (long)n * 384 + (EPI == kEpiQ ? 256 : 0) + co;
+        epi_store<EPI>(im, v, gt, s0[g], s1[g], co, p, HW);
+    }
+}
+
+// 1x1 convolutions as a plain GEMM with register-direct operands (no halo,
+// so nothing is staged in LDS): tile kCoT output channels x 64 R consecutive
+// pixels, wave (wm, wn) = 64 channels x 32 R pixels; every lane loads its
+// 16-byte A (weights) and B (8 channels of one pixel) fragments straight from
+// global memory, two chunks ahead of their MFMAs. R = 4 reads the weights
+// least often; launches that leave CUs idle at that take R = 1, whose
+// epilogue is a quarter as long (gate of one 48x64 image: 17 -> 5.6 us).
+template <int EPI, int R>
 __global__ __launch_bounds__(256) void k_conv1x1(ConvArgs a) {
     __shared__ float bsh[kCoT];  // the tile's biases
     const int HW = a.h * a.w;
@@ -204,9 +364,9 @@ __global__ __launch_bounds__(256) void k_conv1x1(ConvArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
     const int l32 = lane & 31, lhi = lane >> 5;
-    const int p0 = blockIdx.y * 256 + wn * 128;
+    const int p0 = blockIdx.y * (64 * R) + wn * (32 * R);
     const _Float16* wbase = a.wt + ((long)cot * kCoT + wm * 64 + l32) * 16 + lhi * 8;
-    f16x8 A[3][2], B[3][4];
+    f16x8 A[3][2], B[3][R];
     // every load unconditional, from a clamped chunk and pixel (a chunk past
     // the last goes to a slot no step multiplies; a pixel past the map only
     // reaches accumulator columns never stored), so the waits count loads
@@ -221,22 +381,22 @@ __global__ __launch_bounds__(256) void k_conv1x1(ConvArgs a) {
                                    : a.s1.p + (long)n * a.s1.nstride +
                                          (long)(c - a.s0.nchunk) * HW * 16;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
+        for (int r = 0; r < R; r++) {
             const int p = min(p0 + r * 32 + l32, HW - 1);
             B[slot][r] = *reinterpret_cast<const f16x8*>(sp + (long)p * 16 + lhi * 8);
         }
     };
-    f32x16 acc[2][4];
+    f32x16 acc[2][R];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = f32x16{};
+        for (int j = 0; j < R; j++) acc[i][j] = f32x16{};
     // three register slots, so every slot index below is a compile-time constant
     auto step = [&](int c, int slot) {
         load(c + 2, slot == 0 ? 2 : slot - 1);
         if (c < a.nchunk) {  // uniform
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
+            for (int r = 0; r < R; r++) {
                 acc[0][r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[slot][0], B[slot][r],
                                                                    acc[0][r], 0, 0, 0);
                 acc[1][r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[slot][1], B[slot][r],
@@ -252,13 +412,15 @@ __global__ __launch_bounds__(256) void k_conv1x1(ConvArgs a) {
         step(c + 2, 2);
     }
     __syncthreads();  // bsh
+    int p[R];
+    bool in[R];
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int p = p0 + r * 32 + l32;
-        if (p < HW)
-            epi_block<EPI>(a, acc[0][r], acc[1][r], n, cot * kCoT + wm * 64 + 4 * lhi, p, HW,
-                           bsh - cot * kCoT, nullptr);
+    for (int r = 0; r < R; r++) {
+        p[r] = min(p0 + r * 32 + l32, HW - 1);
+        in[r] = p0 + r * 32 + l32 < HW;
     }
+    epi_tile<EPI, 2, R>(a, acc, n, cot * kCoT + wm * 64 + 4 * lhi, p, in, HW, bsh - cot * kCoT,
+                        nullptr);
 }
 
 // The flow encoder's 7x7 stem (4 input channels) with its taps packed into
@@ -345,14 +507,8 @@ __global__ __launch_bounds__(256, 2) void k_conv7p(ConvArgs a) {
             acc[1][r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b, acc[1][r], 0, 0, 0);
         }
     }
-    const int x = tx0 + l32;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int y = ty0 + wn * 4 + r;
-        if (y >= a.h || x >= a.w) continue;
-        epi_block<EPI>(a, acc[0][r], acc[1][r], n, cot * kCoT + wm * 64 + 4 * lhi, y * a.w + x,
-                       HW, bsh - cot * kCoT, nullptr);
-    }
+    epi_rows<EPI, 2, 4>(a, acc, n, cot * kCoT + wm * 64 + 4 * lhi, ty0 + wn * 4, tx0 + l32, HW,
+                        bsh - cot * kCoT, nullptr);
 }
 
 // The 3x3 convolutions: the tile of k_conv7p (kCoT output channels x kTH x kTW
@@ -366,7 +522,10 @@ __global__ __launch_bounds__(256, 2) void k_conv7p(ConvArgs a) {
 // land. 60 KB of LDS: two workgroups a CU. Every staged 32-byte row (a pixel
 // of the patch, an output channel of the weights) has its two 16-byte halves
 // swapped when bit 3 of the row is set, so the 16 lanes of one pass of a
-// 128-bit operand read touch 64 distinct banks.
+// 128-bit operand read touch 64 distinct banks. The input chunks of a long
+// layer with few tiles are split over a.nsplit workgroups (kEpiPart,
+// blockIdx.z = image * nsplit + share; conv_split below), whose sums
+// k_conv_reduce adds in order.
 constexpr int kTH3 = 6;            // output rows of a k_conv3 tile
 constexpr int kPatchUnits = 768;  // 16-byte units of a patch buffer: (kTH + 2) x (kTW + 2) x 2 = 680, padded
 constexpr int kWaTaps = 5, kWbTaps = 4;
@@ -385,7 +544,10 @@ __global__ __launch_bounds__(256, 2) void k_conv3(ConvArgs a) {
     // chunk's barrier
     __shared__ float bsh[kCoT], gsh[kCoT];
     const int HW = a.h * a.w;
-    const int cot = blockIdx.x, tile = blockIdx.y, n = blockIdx.z;
+    const int nsplit = EPI == kEpiPart ? a.nsplit : 1;
+    const int cot = blockIdx.x, tile = blockIdx.y, n = blockIdx.z / nsplit;
+    const int share = blockIdx.z - n * nsplit;
+    const int c_beg = a.nchunk * share / nsplit, c_end = a.nchunk * (share + 1) / nsplit;
     const int ty0 = (tile / a.tiles_x) * TH, tx0 = (tile % a.tiles_x) * kTW;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -450,18 +612,18 @@ __global__ __launch_bounds__(256, 2) void k_conv3(ConvArgs a) {
     // P(1) | WA(1) | WB(1) P(2) | WA(2) ...; a chunk starts once everything
     // issued before it has landed (its patch and WA), its taps 5-8 once WB
     // has (only the next patch, 3 loads, may still be in flight).
-    if (tid < kCoT) bsh[tid] = a.bias[cot * kCoT + tid];
+    if (EPI != kEpiPart && tid < kCoT) bsh[tid] = a.bias[cot * kCoT + tid];
     if constexpr (EPI == kEpiZR || EPI == kEpiQ)
         if (tid < kCoT) gsh[tid] = a.gterm[(long)n * 384 + (EPI == kEpiQ ? 256 : 0) + cot * kCoT + tid];
-    issue_patch(0, 0);
-    issue_w(0, 0, kWaTaps, swa);
-    for (int c = 0; c < nch; c++) {
+    issue_patch(c_beg, c_beg & 1);
+    issue_w(c_beg, 0, kWaTaps, swa);
+    for (int c = c_beg; c < c_end; c++) {
         __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_s_barrier();  // P(c), WA(c) in; every wave done with chunk c - 1
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         issue_w(c, kWaTaps, kWbTaps, swb);
-        const bool more = c + 1 < nch;  // uniform
+        const bool more = c + 1 < c_end;  // uniform
         if (more) issue_patch(c + 1, (c + 1) & 1);
         taps(0, kWaTaps, swa, &sp[c & 1][0]);
         if (more)
@@ -475,14 +637,8 @@ __global__ __launch_bounds__(256, 2) void k_conv3(ConvArgs a) {
         taps(kWaTaps, kWbTaps, swb, &sp[c & 1][0]);
     }
 
-    const int x = tx0 + l32;
-#pragma unroll
-    for (int r = 0; r < RW; r++) {
-        const int y = ty0 + wn * RW + r;
-        if (y >= a.h || x >= a.w) continue;
-        epi_block<EPI>(a, acc[0][r], acc[1][r], n, cot * kCoT + wm * 64 + 4 * lhi, y * a.w + x,
-                       HW, bsh - cot * kCoT, gsh - cot * kCoT);
-    }
+    epi_rows<EPI, 2, RW>(a, acc, EPI == kEpiPart ? (int)blockIdx.z : n, cot * kCoT + wm * 64 + 4 * lhi, ty0 + wn * RW, tx0 + l32, HW,
+                         bsh - cot * kCoT, gsh - cot * kCoT);
 }
 
 // NCHW fp32 [image][C][hw] -> CK fp16 chunks [c0 ..) of out; channels past C
@@ -519,42 +675,57 @@ __global__ __launch_bounds__(256) void k_to_ck(const float* in, long in_nstride,
 // fixed-order tree over the threads.
 __global__ __launch_bounds__(256) void k_gate_pool(const _Float16* gate, long nstride, int hw,
                                                    float* glo) {
-    __shared__ float red[256][17];
+    __shared__ float red[4][16];
     const int n = blockIdx.y, ch = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const _Float16* g = gate + (long)n * nstride + (long)ch * hw * 16;
     float s[16] = {};
-    for (int p = threadIdx.x; p < hw; p += 256) {
-        const f16x8 a = *reinterpret_cast<const f16x8*>(g + (long)p * 16);
-        const f16x8 b = *reinterpret_cast<const f16x8*>(g + (long)p * 16 + 8);
+    // four pixels' loads in flight, from a clamped pixel, masked after
+    for (int p0 = threadIdx.x; p0 < hw; p0 += 1024) {
+        f16x8 v[4][2];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            s[i] += (float)a[i];
-            s[8 + i] += (float)b[i];
+        for (int u = 0; u < 4; u++) {
+            const _Float16* q = g + (long)min(p0 + 256 * u, hw - 1) * 16;
+            v[u][0] = *reinterpret_cast<const f16x8*>(q);
+            v[u][1] = *reinterpret_cast<const f16x8*>(q + 8);
         }
-    }
 #pragma unroll
-    for (int i = 0; i < 16; i++) red[threadIdx.x][i] = s[i];
+        for (int u = 0; u < 4; u++)
+            if (p0 + 256 * u < hw)
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    s[i] += (float)v[u][0][i];
+                    s[8 + i] += (float)v[u][1][i];
+                }
+    }
+    int base, valid;
+    wave_reduce_scatter(s, lane, base, valid);
+    if (valid > 0) red[wave][base] = s[0];  // 16 values over 64 lanes: at most one a lane
     __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if (threadIdx.x < st)
-#pragma unroll
-            for (int i = 0; i < 16; i++) red[threadIdx.x][i] += red[threadIdx.x + st][i];
-        __syncthreads();
+    if (threadIdx.x < 16) {
+        const int i = threadIdx.x;
+        glo[(long)n * 128 + ch * 16 + i] =
+            ((red[0][i] + red[1][i]) + (red[2][i] + red[3][i])) / (float)hw;
     }
-    if (threadIdx.x < 16) glo[(long)n * 128 + ch * 16 + threadIdx.x] = red[0][threadIdx.x] / (float)hw;
 }
 
 // The three 1x1 global convolutions of the pooled vector (convz_glo,
-// convr_glo, convq_glo, main.cu:492-523): gterm[n][j] = round16(W[j] .
-// round16(glo[n]) + b[j]) for j in 0..383, W and b stacked z | r | q.
-__global__ __launch_bounds__(384) void k_glo_fc(const float* glo, const float* W, const float* b,
+// convr_glo, convq_glo, main.cu:492-523): gterm[n][j] = round16(W[.][j] .
+// round16(glo[n]) + b[j]) for j in 0..383, W [128][384] and b stacked z | r | q
+// by columns, one workgroup per image and layer, a column per thread with all
+// its loads in flight (one workgroup per image reading rows took 7.2 us).
+__global__ __launch_bounds__(128) void k_glo_fc(const float* glo, const float* W, const float* b,
                                                 float* gterm) {
     __shared__ float gs[128];
-    const int n = blockIdx.x, j = threadIdx.x;
-    if (j < 128) gs[j] = r16(glo[(long)n * 128 + j]);
+    const int n = blockIdx.x, j = blockIdx.y * 128 + threadIdx.x;
+    float w[128];
+#pragma unroll
+    for (int c = 0; c < 128; c++) w[c] = W[c * 384 + j];
+    gs[threadIdx.x] = r16(glo[(long)n * 128 + threadIdx.x]);
     __syncthreads();
     float s = 0.0f;
-    for (int c = 0; c < 128; c++) s += W[(long)j * 128 + c] * gs[c];
+#pragma unroll
+    for (int c = 0; c < 128; c++) s += w[c] * gs[c];
     gterm[(long)n * 384 + j] = r16(s + b[j]);
 }
 
@@ -773,9 +944,13 @@ struct UpdateState {
     // caller's stream: forked by ev_fork, joined by ev_join before convz|convr
     hipStream_t side[2] = {nullptr, nullptr};
     hipEvent_t ev_fork = nullptr, ev_join[2] = {nullptr, nullptr};
-    // motion filter (batch 1): grid coords, lookup, motion, state copies, heads
-    DevBuf mf_coords, mf_corr, mf_motion, mf_net, mf_inp, mf_delta, mf_weight, mf_agg;
-    std::vector<float> mf_host;
+    // motion filter (batch 1): grid coords, lookup, motion, new state, heads;
+    // delta on the host
+    DevBuf mf_coords, mf_corr, mf_motion, mf_net, mf_delta, mf_weight, mf_agg;
+    HostStage mf_host;
+    bool mf_ready = false;
+    DevBuf part;  // sums of split convolutions (convz|convr, convq; the caller's stream only)
+    int cus = 0;
     int tiles_x = 0, tiles_y = 0;
 };
 
@@ -885,10 +1060,12 @@ int pack_all(UpdateState* s) {
     SLK_TRY(pack(s->q, s, {L_Q}));
     SLK_TRY(pack(s->heads, s, {L_DL0, L_WT0, L_AG1}));
     SLK_TRY(pack(s->ag2, s, {L_AG2}));
-    // global convs: [384][128] rounded, stacked z | r | q
-    std::vector<float> gw, gb;
+    // global convs: [128 inputs][384 outputs] rounded, outputs stacked z | r | q
+    std::vector<float> gw(128 * 384), gb;
+    int col = 0;
     for (int L : {L_ZG, L_RG, L_QG}) {
-        gw.insert(gw.end(), s->hw_[L].begin(), s->hw_[L].end());
+        for (int o = 0; o < 128; o++, col++)
+            for (int c = 0; c < 128; c++) gw[c * 384 + col] = s->hw_[L][o * 128 + c];
         gb.insert(gb.end(), s->hb_[L].begin(), s->hb_[L].end());
     }
     SLK_TRY(upload_rounded(s->glo_w, gw));
@@ -909,6 +1086,27 @@ int pack_all(UpdateState* s) {
     return SLK_OK;
 }
 
+// Workgroups that share the input chunks of a 28-chunk 3x3 convolution of wgs
+// tiles. A lone workgroup on a CU takes 1.8 us a chunk and two together 3.5 us
+// (the loads, products and barriers of one chunk are a serial chain), so a
+// launch that leaves CUs idle is as long as its chunks are many; a split costs
+// a pass over its sums, about 6 us. The share of least estimated time, at
+// least four chunks of it, while all workgroups stay resident; none from two
+// workgroups a CU on. One 48x64 image (32 and 16 tiles, seven shares):
+// convz|convr 45 -> 19.6 us, convq 52 -> 21 us, both passes.
+int conv_split(int cus, long wgs, int nchunk) {
+    int best = 1;
+    float least = 0.0f;
+    for (int k = 1; k <= nchunk / 4 && (k == 1 || wgs * k <= 2L * cus); k++) {
+        const float t = (float)((nchunk + k - 1) / k) * (wgs * k > cus ? 3.5f : 1.8f) + (k > 1 ? 6.0f : 0.0f);
+        if (k == 1 || t < least) {
+            best = k;
+            least = t;
+        }
+    }
+    return wgs >= 2L * cus ? 1 : best;
+}
+
 template <int KS, int EPI>
 int launch_conv(const UpdateState* s, const PackedConv& pc, ConvArgs a, int N,
                 hipStream_t stream) {
@@ -922,14 +1120,33 @@ int launch_conv(const UpdateState* s, const PackedConv& pc, ConvArgs a, int N,
     a.tiles_x = s->tiles_x;
     if (a.s0.nchunk > a.nchunk) a.s0.nchunk = a.nchunk;
     if constexpr (KS == 1) {
-        const int hw = s->h * s->w;
-        hipLaunchKernelGGL((k_conv1x1<EPI>), dim3(pc.co_tot / kCoT, (hw + 255) / 256, N),
-                           dim3(256), 0, stream, a);
+        const int hw = s->h * s->w, cot = pc.co_tot / kCoT;
+        // the wide tile once it gives every CU a workgroup
+        if ((long)cot * ((hw + 255) / 256) * N >= s->cus)
+            hipLaunchKernelGGL((k_conv1x1<EPI, 4>), dim3(cot, (hw + 255) / 256, N), dim3(256), 0,
+                               stream, a);
+        else
+            hipLaunchKernelGGL((k_conv1x1<EPI, 1>), dim3(cot, (hw + 63) / 64, N), dim3(256), 0,
+                               stream, a);
     } else if constexpr (KS == 3) {
         a.zero16 = s->zero16.as<_Float16>();
-        const int ty = (s->h + kTH3 - 1) / kTH3;
-        hipLaunchKernelGGL((k_conv3<EPI, kTH3>), dim3(pc.co_tot / kCoT, s->tiles_x * ty, N),
-                           dim3(256), 0, stream, a);
+        const int tiles = s->tiles_x * ((s->h + kTH3 - 1) / kTH3), cot = pc.co_tot / kCoT;
+        const long wgs = (long)cot * tiles * N;
+        if constexpr (EPI == kEpiZR || EPI == kEpiQ) {
+            const int split = conv_split(s->cus, wgs, a.nchunk);
+            if (split > 1) {
+                a.part = s->part.template as<float>();
+                a.nsplit = split;
+                hipLaunchKernelGGL((k_conv3<kEpiPart, kTH3>), dim3(cot, tiles, N * split), dim3(256),
+                                   0, stream, a);
+                SLK_HIP(hipGetLastError());
+                hipLaunchKernelGGL((k_conv_reduce<EPI>), dim3((s->h * s->w + 63) / 64, pc.Co / 16, N),
+                                   dim3(64), 0, stream, a);
+                SLK_HIP(hipGetLastError());
+                return SLK_OK;
+            }
+        }
+        hipLaunchKernelGGL((k_conv3<EPI, kTH3>), dim3(cot, tiles, N), dim3(256), 0, stream, a);
     } else {
         static_assert(KS == 7, "the 7x7 stem is the only other convolution");
         hipLaunchKernelGGL((k_conv7p<EPI>), dim3(pc.co_tot / kCoT, s->tiles_x * s->tiles_y, N),
@@ -976,7 +1193,21 @@ extern "C" int slk_update_create(slk_update** out, int max_batch, int h, int w) 
     s.tiles_y = (h + kTH - 1) / kTH;
     const size_t hw = (size_t)h * w, chunk = hw * 16 * sizeof(_Float16);
     const size_t N = (size_t)max_batch;
-    int st = SLK_OK;
+    int st = SLK_OK, dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        st = fail(SLK_E_HIP, "update_create: device attributes failed");
+    if (st == SLK_OK) {
+        // the largest sums of any batch: co_tot channels of split * batch images
+        const int tiles = s.tiles_x * ((h + kTH3 - 1) / kTH3);
+        size_t most = 0;
+        for (int b = 1; b <= max_batch && (long)b * tiles < 2L * s.cus; b++)
+            for (int cot = 1; cot <= 2; cot++) {
+                const int split = conv_split(s.cus, (long)cot * tiles * b, kCatCh);
+                if (split > 1) most = std::max(most, (size_t)split * b * cot * kCoT * hw);
+            }
+        if (most) st = s.part.ensure(most * sizeof(float));
+    }
     if (st == SLK_OK) st = s.corr16.ensure(N * kCorrCh * chunk);
     if (st == SLK_OK) st = s.mot16.ensure(N * chunk);
     if (st == SLK_OK) st = s.cat.ensure(N * kCatCh * chunk);
@@ -1022,10 +1253,11 @@ extern "C" int slk_update_destroy(slk_update* u) {
     for (DevBuf* b : {&s.glo_w, &s.glo_b, &s.small_w[0], &s.small_w[1], &s.small_w[2],
                       &s.small_b[0], &s.small_b[1], &s.small_b[2], &s.corr16, &s.mot16, &s.cat,
                       &s.tmp, &s.tmp_f, &s.tmp_g, &s.zr_buf, &s.glo, &s.gterm, &s.agg16, &s.agg_t,
-                      &s.zero16, &s.mf_coords,
-                      &s.mf_corr, &s.mf_motion, &s.mf_net, &s.mf_inp, &s.mf_delta, &s.mf_weight,
+                      &s.zero16, &s.part, &s.mf_coords,
+                      &s.mf_corr, &s.mf_motion, &s.mf_net, &s.mf_delta, &s.mf_weight,
                       &s.mf_agg})
         b->release();
+    s.mf_host.release();
     delete u;
     return SLK_OK;
 }
@@ -1090,55 +1322,31 @@ extern "C" int slk_update_load_dir(slk_update* u, const char* dir) {
     return SLK_OK;
 }
 
-extern "C" int slk_update_forward(slk_update* u, const float* corr, const float* motion,
-                                  float* net, const float* inp, float* delta_out,
-                                  float* weight_out, float* agg_conv1_out, int batch,
-                                  hipStream_t stream) {
-    if (!u) return fail(SLK_E_ARG, "update_forward: null module");
-    UpdateState& s = u->s;
-    if (batch < 0 || batch > s.max_batch)
-        return fail(SLK_E_ARG, "update_forward: batch outside [0, max_batch]");
-    if (batch == 0) return SLK_OK;
-    if (!corr || !motion || !net || !inp || !delta_out || !weight_out || !agg_conv1_out)
-        return fail(SLK_E_ARG, "update_forward: null argument");
-    if (!s.packed) SLK_TRY(pack_all(&s));
-    const int hw = s.h * s.w, N = batch;
+namespace {
+
+// NCHW fp32 channels to chunks c0 .. of a CK buffer of out_ch chunks an image
+void to_ck(const float* in, int C, const DevBuf& out, int out_ch, int c0, int hw, int N,
+           hipStream_t on) {
+    hipLaunchKernelGGL(k_to_ck<false>, dim3((hw + 255) / 256, (C + 15) / 16, N), dim3(256), 0, on,
+                       in, (long)C * hw, C, out.as<_Float16>(), (long)out_ch * hw * 16, c0, hw,
+                       nullptr);
+}
+
+// The parts of a forward step that do not need the correlation: the flow
+// encoder on side[0] and the gate on side[1], after ev_fork and left to
+// forward_gru to join. The caller records ev_fork on its stream first: it
+// follows everything queued there before (the inputs, and the previous call's
+// readers of cat and the scratch).
+int forward_sides(UpdateState& s, const float* motion, const float* net, const float* inp, int N) {
+    const int hw = s.h * s.w;
     const long ck = (long)hw * 16;  // elements of one chunk
-    // inputs to CK fp16: corr (196 ch), motion (4 ch), net and inp (128 ch)
-    auto to_ck = [&](const float* in, int C, DevBuf& out, int out_ch, int c0, float* wb,
-                     hipStream_t on) {
-        dim3 g((hw + 255) / 256, (C + 15) / 16, N);
-        hipLaunchKernelGGL(k_to_ck<false>, g, dim3(256), 0, on, in, (long)C * hw, C,
-                           out.as<_Float16>(), out_ch * ck, c0, hw, wb);
-    };
-    const long catS = kCatCh * ck, tmpS = kTmpCh * ck, zrS = kZrCh * ck;
-    // The three encoders of convz|convr's input are independent: the flow
-    // encoder runs on side[0], the gate on side[1], the correlation encoder on
-    // the caller's stream; each writes its own chunks of cat through its own
-    // scratch, and the caller's stream waits for both sides before convz|convr.
-    // The fork follows everything the caller queued before this call (the
-    // inputs, and the previous call's readers of cat and the scratch).
+    const long catS = kCatCh * ck, tmpS = kTmpCh * ck;
     hipStream_t sf = s.side[0], sg = s.side[1];
-    SLK_HIP(hipEventRecord(s.ev_fork, stream));
     SLK_HIP(hipStreamWaitEvent(sf, s.ev_fork, 0));
     SLK_HIP(hipStreamWaitEvent(sg, s.ev_fork, 0));
-    // corr encoder: 1x1 196 -> 128, 3x3 128 -> 128 into cat chunks 16..23
-    {
-        to_ck(corr, 196, s.corr16, kCorrCh, 0, nullptr, stream);
-        ConvArgs a{};
-        a.s0 = src(s.corr16, 0, kCorrCh, kCorrCh * ck, hw);
-        a.out16 = s.tmp.as<_Float16>();
-        a.out16_nstride = tmpS;
-        SLK_TRY((launch_conv<1, kEpiRelu>(&s, s.ce0, a, N, stream)));
-        ConvArgs b{};
-        b.s0 = src(s.tmp, 0, 8, tmpS, hw);
-        b.out16 = s.cat.as<_Float16>() + 16 * ck;
-        b.out16_nstride = catS;
-        SLK_TRY((launch_conv<3, kEpiRelu>(&s, s.ce2, b, N, stream)));
-    }
     // flow encoder: 7x7 4 -> 128, 3x3 128 -> 64 into cat chunks 24..27
     {
-        to_ck(motion, 4, s.mot16, 1, 0, nullptr, sf);
+        to_ck(motion, 4, s.mot16, 1, 0, hw, N, sf);
         ConvArgs a{};
         a.s0 = src(s.mot16, 0, 1, ck, hw);
         a.out16 = s.tmp_f.as<_Float16>();
@@ -1154,8 +1362,8 @@ extern "C" int slk_update_forward(slk_update* u, const float* corr, const float*
     // net and inp into cat chunks 0..15; GRU gate = round16(sigmoid(w(net)))
     // * net, pooled; global terms
     {
-        to_ck(net, 128, s.cat, kCatCh, 0, nullptr, sg);
-        to_ck(inp, 128, s.cat, kCatCh, 8, nullptr, sg);
+        to_ck(net, 128, s.cat, kCatCh, 0, hw, N, sg);
+        to_ck(inp, 128, s.cat, kCatCh, 8, hw, N, sg);
         ConvArgs a{};
         a.s0 = src(s.cat, 0, 8, catS, hw);
         a.out16 = s.tmp_g.as<_Float16>();
@@ -1165,11 +1373,38 @@ extern "C" int slk_update_forward(slk_update* u, const float* corr, const float*
         SLK_TRY((launch_conv<1, kEpiGate>(&s, s.gw, a, N, sg)));
         hipLaunchKernelGGL(k_gate_pool, dim3(8, N), dim3(256), 0, sg, s.tmp_g.as<_Float16>(),
                            tmpS, hw, s.glo.as<float>());
-        hipLaunchKernelGGL(k_glo_fc, dim3(N), dim3(384), 0, sg, s.glo.as<float>(),
+        hipLaunchKernelGGL(k_glo_fc, dim3(N, 3), dim3(128), 0, sg, s.glo.as<float>(),
                            s.glo_w.as<float>(), s.glo_b.as<float>(), s.gterm.as<float>());
         SLK_HIP(hipGetLastError());
         SLK_HIP(hipEventRecord(s.ev_join[1], sg));
     }
+    return SLK_OK;
+}
+
+// corr encoder: 1x1 196 -> 128, 3x3 128 -> 128 into cat chunks 16..23
+int forward_corr(UpdateState& s, const float* corr, int N, hipStream_t stream) {
+    const int hw = s.h * s.w;
+    const long ck = (long)hw * 16, catS = kCatCh * ck, tmpS = kTmpCh * ck;
+    to_ck(corr, 196, s.corr16, kCorrCh, 0, hw, N, stream);
+    ConvArgs a{};
+    a.s0 = src(s.corr16, 0, kCorrCh, kCorrCh * ck, hw);
+    a.out16 = s.tmp.as<_Float16>();
+    a.out16_nstride = tmpS;
+    SLK_TRY((launch_conv<1, kEpiRelu>(&s, s.ce0, a, N, stream)));
+    ConvArgs b{};
+    b.s0 = src(s.tmp, 0, 8, tmpS, hw);
+    b.out16 = s.cat.as<_Float16>() + 16 * ck;
+    b.out16_nstride = catS;
+    SLK_TRY((launch_conv<3, kEpiRelu>(&s, s.ce2, b, N, stream)));
+    return SLK_OK;
+}
+
+// The rest of a forward step on the caller's stream once the sides and the
+// corr encoder are done: the GRU (its new state to net_out) and the heads.
+int forward_gru(UpdateState& s, float* net_out, float* delta_out, float* weight_out,
+                float* agg_conv1_out, int N, hipStream_t stream) {
+    const int hw = s.h * s.w;
+    const long ck = (long)hw * 16, catS = kCatCh * ck, zrS = kZrCh * ck;
     SLK_HIP(hipStreamWaitEvent(stream, s.ev_join[0], 0));
     SLK_HIP(hipStreamWaitEvent(stream, s.ev_join[1], 0));
     // z | r (one 256-row GEMM over the 448-channel concatenation), then q and
@@ -1192,7 +1427,7 @@ extern "C" int slk_update_forward(slk_update* u, const float* corr, const float*
         b.net16 = s.cat.as<_Float16>();
         b.net_nstride = catS;
         b.gterm = s.gterm.as<float>();
-        b.out32 = net;
+        b.out32 = net_out;
         b.out32_nstride = 128L * hw;
         SLK_TRY((launch_conv<3, kEpiQ>(&s, s.q, b, N, stream)));
     }
@@ -1226,6 +1461,29 @@ extern "C" int slk_update_forward(slk_update* u, const float* corr, const float*
         SLK_HIP(hipGetLastError());
     }
     return SLK_OK;
+}
+
+}  // namespace
+
+extern "C" int slk_update_forward(slk_update* u, const float* corr, const float* motion,
+                                  float* net, const float* inp, float* delta_out,
+                                  float* weight_out, float* agg_conv1_out, int batch,
+                                  hipStream_t stream) {
+    if (!u) return fail(SLK_E_ARG, "update_forward: null module");
+    UpdateState& s = u->s;
+    if (batch < 0 || batch > s.max_batch)
+        return fail(SLK_E_ARG, "update_forward: batch outside [0, max_batch]");
+    if (batch == 0) return SLK_OK;
+    if (!corr || !motion || !net || !inp || !delta_out || !weight_out || !agg_conv1_out)
+        return fail(SLK_E_ARG, "update_forward: null argument");
+    if (!s.packed) SLK_TRY(pack_all(&s));
+    // The three encoders of convz|convr's input are independent: the flow
+    // encoder and the gate run beside the correlation encoder, each writing
+    // its own chunks of cat through its own scratch.
+    SLK_HIP(hipEventRecord(s.ev_fork, stream));
+    SLK_TRY(forward_corr(s, corr, batch, stream));
+    SLK_TRY(forward_sides(s, motion, net, inp, batch));
+    return forward_gru(s, net, delta_out, weight_out, agg_conv1_out, batch, stream);
 }
 
 extern "C" int slk_update_compute_eta(slk_update* u, float* agg_features, float* eta_out,
@@ -1283,37 +1541,42 @@ extern "C" int slk_motion_filter(slk_ctx* ctx, slk_update* u, const void* f_last
     if (ctx->levels != 4) return fail(SLK_E_ARG, "motion_filter: needs a 4-level context");
     const int hw = s.h * s.w;
     const size_t f4 = sizeof(float);
-    if (!s.mf_coords.ptr) {
+    if (!s.packed) SLK_TRY(pack_all(&s));
+    if (!s.mf_ready) {
         SLK_TRY(s.mf_coords.ensure(2 * hw * f4));
         SLK_TRY(s.mf_corr.ensure(196 * hw * f4));
         SLK_TRY(s.mf_motion.ensure(4 * hw * f4));
         SLK_TRY(s.mf_net.ensure(128 * hw * f4));
-        SLK_TRY(s.mf_inp.ensure(128 * hw * f4));
         SLK_TRY(s.mf_delta.ensure(3 * hw * f4));
         SLK_TRY(s.mf_weight.ensure(3 * hw * f4));
         SLK_TRY(s.mf_agg.ensure(128 * hw * f4));
-        s.mf_host.resize(2 * (size_t)hw);
+        SLK_TRY(s.mf_host.ensure(2 * hw * f4));
+        // the identity grid and the zero motion, which no call writes again
+        SLK_TRY(slk_fill_coords0(s.mf_coords.as<float>(), 1, s.h, s.w, stream));
+        SLK_HIP(hipMemsetAsync(s.mf_motion.ptr, 0, 4 * hw * f4, stream));
+        SLK_HIP(hipStreamSynchronize(stream));
+        s.mf_ready = true;
     }
-    // build_correlation(last_kf, temp slot) and the lookup at the identity
-    // grid (main.cu:1939-1951)
+    // build_correlation(last_kf, temp slot) and the lookup at the identity grid
+    // (main.cu:1939-1951), then beside them the parts that only need the
+    // keyframe's hidden state and context and zero motion (main.cu:1954-1961);
+    // the new state goes to a buffer of its own, the keyframe's stays
+    SLK_HIP(hipEventRecord(s.ev_fork, stream));
     SLK_TRY(slk_corr_build(ctx, f_last, f_cur, dtype, stream));
-    SLK_TRY(slk_fill_coords0(s.mf_coords.as<float>(), 1, s.h, s.w, stream));
     SLK_TRY(slk_corr_sample(ctx, s.mf_coords.as<float>(), s.mf_corr.as<float>(), stream));
-    // the keyframe's hidden state and context, zero motion (main.cu:1954-1961)
-    SLK_HIP(hipMemcpyAsync(s.mf_net.ptr, net_kf, 128 * hw * f4, hipMemcpyDeviceToDevice, stream));
-    SLK_HIP(hipMemcpyAsync(s.mf_inp.ptr, inp_kf, 128 * hw * f4, hipMemcpyDeviceToDevice, stream));
-    SLK_HIP(hipMemsetAsync(s.mf_motion.ptr, 0, 4 * hw * f4, stream));
-    SLK_TRY(slk_update_forward(u, s.mf_corr.as<float>(), s.mf_motion.as<float>(),
-                               s.mf_net.as<float>(), s.mf_inp.as<float>(), s.mf_delta.as<float>(),
-                               s.mf_weight.as<float>(), s.mf_agg.as<float>(), 1, stream));
+    SLK_TRY(forward_sides(s, s.mf_motion.as<float>(), net_kf, inp_kf, 1));
+    SLK_TRY(forward_corr(s, s.mf_corr.as<float>(), 1, stream));
+    SLK_TRY(forward_gru(s, s.mf_net.as<float>(), s.mf_delta.as<float>(), s.mf_weight.as<float>(),
+                        s.mf_agg.as<float>(), 1, stream));
     // mean flow magnitude of delta's first two channels, summed on the host in
     // pixel order as the reference does (main.cu:1970-1981)
-    SLK_HIP(hipMemcpyAsync(s.mf_host.data(), s.mf_delta.ptr, 2 * hw * f4, hipMemcpyDeviceToHost,
+    const float* d = static_cast<const float*>(s.mf_host.ptr);
+    SLK_HIP(hipMemcpyAsync(s.mf_host.ptr, s.mf_delta.ptr, 2 * hw * f4, hipMemcpyDeviceToHost,
                            stream));
     SLK_HIP(hipStreamSynchronize(stream));
     float sum = 0.0f;
     for (int k = 0; k < hw; k++) {
-        const float dx = s.mf_host[k], dy = s.mf_host[hw + k];
+        const float dx = d[k], dy = d[hw + k];
         sum += std::sqrt(dx * dx + dy * dy);
     }
     *mean_flow = sum / (float)hw;

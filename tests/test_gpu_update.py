@@ -98,6 +98,24 @@ def test_update_window_48_edges(slk):
     check(g["eta"][[0, 5, 11]], re, "eta")
 
 
+@pytest.mark.parametrize("n,h,w", [(1, 3, 5), (1, 20, 33), (3, 48, 64), (9, 48, 64), (15, 48, 64),
+                                   (16, 48, 64), (21, 48, 64), (22, 48, 64)])
+def test_update_few_edges(slk, n, h, w):
+    """Batches that leave compute units idle take split convolutions (their
+    channel shares summed by a second kernel) and narrow 1x1 tiles: the
+    smallest map, a ragged one, the share counts between one edge and the last
+    split batch, and both sides of the 1x1 rule (256 / 12 tiles an edge). The
+    last edge is checked, alone in the oracle (edges are independent); the
+    shares are added in fp32, so the file's bar holds."""
+    announce(f"update operator {n} edges {h}x{w}")
+    P = uo.seeded_weights(40)
+    corr, motion, net, inp = uo.seeded_inputs(n, h, w, seed=41 + n)
+    g = run_gpu(slk, P, corr, motion, net, inp)
+    refs = uo.update_forward(P, corr[-1:], motion[-1:], net[-1:], inp[-1:])
+    for name, ref in zip(("net", "delta", "weight", "agg"), refs):
+        check(g[name][-1:], ref, f"{name} {n}x{h}x{w}")
+
+
 def test_weights_from_reference_tensor_files(slk, tmp_path):
     """slk_update_load_dir reads the reference's exported tensor files
     (<name>_weight.bin / _bias.bin: int32 ndim, dims, float32 data) and gives
