@@ -131,32 +131,53 @@ __global__ __launch_bounds__(256) void k_rows(float* __restrict__ dst,
         reinterpret_cast<V*>(d)[i] = reinterpret_cast<const V*>(s)[i];
 }
 
-// Keyframe means: csr = [na + 1 offsets][edge ids grouped by keyframe, edge
-// order within a group]; dst row a = sum of its rows from zero, in that
-// order, then fma(1/count - 1, S, S) when count > 1.
-template <int kV>
+// Index lists of a call: in the launch's arguments while they fit (kArgInts, half
+// of the 4 KiB that a launch takes; a 48-edge window has 73), else in the
+// uploaded buffer. An upload and the copy of the active list out of it were two
+// 4 us copies and an event a call (mean and eta of a 48x64 window: 58.7 us with
+// them, 51.9 without).
+constexpr int kArgInts = 512;
+struct ArgList {
+    int v[kArgInts];
+    __device__ __forceinline__ int operator[](int i) const { return v[i]; }
+};
+struct MemList {
+    const int* v;
+    __device__ __forceinline__ int operator[](int i) const { return v[i]; }
+};
+
+// Keyframe means: csr = [na + 1 offsets][n edge ids grouped by keyframe, edge
+// order within a group][na keyframes]; dst row a = sum of its rows from zero,
+// in that order (four rows' loads in flight), then fma(1/count - 1, S, S) when
+// count > 1; the keyframes go to active_kf.
+template <int kV, class L>
 __global__ __launch_bounds__(256) void k_scatter_mean(float* __restrict__ dst,
-                                                      const float* __restrict__ src,
-                                                      const int* __restrict__ csr, int na,
-                                                      long row) {
+                                                      const float* __restrict__ src, L csr, int na,
+                                                      int n, long row,
+                                                      int* __restrict__ active_kf) {
     using V = typename std::conditional<kV == 4, float4, float>::type;
     const int a = blockIdx.y;
     const int b0 = csr[a], b1 = csr[a + 1];
-    const int* ed = csr + na + 1;
     const int count = b1 - b0;
     const float inv = 1.0f / (float)count;
     const long nv = row / kV;
+    if (active_kf && blockIdx.x == 0 && threadIdx.x == 0) active_kf[a] = csr[na + 1 + n + a];
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < nv;
          i += (long)gridDim.x * blockDim.x) {
         float acc[kV];
 #pragma unroll
         for (int j = 0; j < kV; j++) acc[j] = 0.0f;
-        for (int b = b0; b < b1; b++) {
-            float x[kV];
-            *reinterpret_cast<V*>(x) =
-                reinterpret_cast<const V*>(src + (long)ed[b] * row)[i];
+        for (int b = b0; b < b1; b += 4) {
+            float x[4][kV];
 #pragma unroll
-            for (int j = 0; j < kV; j++) acc[j] = acc[j] + x[j];
+            for (int q = 0; q < 4; q++)
+                *reinterpret_cast<V*>(x[q]) = reinterpret_cast<const V*>(
+                    src + (long)csr[na + 1 + min(b + q, b1 - 1)] * row)[i];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (b + q < b1)  // uniform
+#pragma unroll
+                    for (int j = 0; j < kV; j++) acc[j] = acc[j] + x[q][j];
         }
         if (count > 1) {
 #pragma unroll
@@ -332,18 +353,28 @@ extern "C" int slk_scatter_mean(slk_ctx* ctx, float* dst, const float* src, cons
     std::fill(fill.begin(), fill.end(), 0);
     for (int e = 0; e < n; e++) ed[off[slot[e]] + fill[slot[e]]++] = e;
     std::copy(act.begin(), act.end(), ed + n);
-    SLK_TRY(upload(ctx, buf.data(), buf.size() * sizeof(int), stream));
-    const int* csr = ctx->glue_idx.as<int>();
-    if (row % 4 == 0 && al16(dst) && al16(src))
-        hipLaunchKernelGGL(k_scatter_mean<4>, row_grid(row / 4, na), dim3(256), 0, stream, dst,
-                           src, csr, na, row);
-    else
-        hipLaunchKernelGGL(k_scatter_mean<1>, row_grid(row, na), dim3(256), 0, stream, dst, src,
-                           csr, na, row);
+    const bool v4 = row % 4 == 0 && al16(dst) && al16(src);
+    const dim3 grid = row_grid(v4 ? row / 4 : row, na);
+    if (buf.size() <= (size_t)kArgInts) {
+        ArgList l;
+        std::copy(buf.begin(), buf.end(), l.v);
+        if (v4)
+            hipLaunchKernelGGL((k_scatter_mean<4, ArgList>), grid, dim3(256), 0, stream, dst, src, l,
+                               na, n, row, active_kf);
+        else
+            hipLaunchKernelGGL((k_scatter_mean<1, ArgList>), grid, dim3(256), 0, stream, dst, src, l,
+                               na, n, row, active_kf);
+    } else {
+        SLK_TRY(upload(ctx, buf.data(), buf.size() * sizeof(int), stream));
+        const MemList l{ctx->glue_idx.as<int>()};
+        if (v4)
+            hipLaunchKernelGGL((k_scatter_mean<4, MemList>), grid, dim3(256), 0, stream, dst, src, l,
+                               na, n, row, active_kf);
+        else
+            hipLaunchKernelGGL((k_scatter_mean<1, MemList>), grid, dim3(256), 0, stream, dst, src, l,
+                               na, n, row, active_kf);
+    }
     SLK_HIP(hipGetLastError());
-    if (active_kf)
-        SLK_HIP(hipMemcpyAsync(active_kf, csr + na + 1 + n, na * sizeof(int),
-                               hipMemcpyDeviceToDevice, stream));
     if (active_kf_host) std::copy(act.begin(), act.end(), active_kf_host);
     *num_active_host = na;
     return SLK_OK;

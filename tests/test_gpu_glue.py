@@ -184,6 +184,23 @@ def test_scatter_mean_backend_counts(slk, ctx):
     np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("n", [491, 492])
+@pytest.mark.parametrize("row", [16, 61])
+def test_scatter_mean_list_sizes(slk, ctx, n, row):
+    """512 and 513 list entries (10 keyframes: 2 * 10 + 1 + n): the last list
+    that goes with the launch and the first that is uploaded; counts with every
+    remainder of 4, from 1 edge on."""
+    rng = np.random.default_rng(17)
+    counts = np.array([1, 2, 3, 4, 5, 6, 7, 8, 9, n - 45])
+    ii = rng.permutation(np.repeat(3 * np.arange(10), counts)).astype(np.int32)
+    src = rng.normal(0, 100, size=(n, row)).astype(np.float32)
+    got, act_d, act_h = _scatter_mean(slk, ctx, src, ii)
+    ref, act = orc.scatter_mean(src, ii)
+    np.testing.assert_array_equal(act_h, act)
+    np.testing.assert_array_equal(act_d, act)
+    np.testing.assert_array_equal(got, ref)
+
+
 def test_ba_edge_set(slk, ctx):
     announce("glue ba_edge_set")
     L = slk.lib()
