@@ -10,11 +10,10 @@
 //    v_mfma_f32_32x32x16_f16 and the epilogue applies both roundings;
 //  * instance norm (instance_norm_half_kernel, nn.cuh:609-654): mean and
 //    variance over the h*w pixels of one channel of fp16 data in fp32, eps
-//    1e-5, result rounded to fp16. Here a statistics kernel writes per-split
-//    (mean, M2) pairs and the normalising kernel combines them (the total
-//    mean from the split means, then M2 = sum of the splits' M2 plus their
-//    count-weighted squared mean offsets) before it applies the norm, the
-//    ReLU and the residual add of the block in one pass;
+//    1e-5, result rounded to fp16. Here the convolution leaves a (mean, M2)
+//    pair per tile and channel in fp32 and the normalising kernel combines
+//    them in double before it applies the norm, the ReLU and the residual add
+//    of the block in one pass;
 //  * ReLU and the residual add of fp16 values (relu_half_kernel,
 //    add_half_kernel, nn.cuh:588-607) are exact / one rounding.
 //
@@ -30,6 +29,7 @@
 #include <string>
 #include <vector>
 
+#include "reduce.hpp"
 #include "slk_internal.hpp"
 
 namespace slk {
@@ -49,6 +49,17 @@ enum EncEpi {
     kEpAddRelu = 2,  // relu(round16(relu(y) + res)), res a CK tensor of the output shape
     kEpNchw = 3,     // y to an NCHW fp16 output (the encoder's result)
     kEpNetInp = 4,   // channels < 128: net = tanh(y); the rest: inp = relu(y), NCHW fp32
+    kEpStats = 5,    // kEpRaw, and the tile's statistics for an instance norm
+};
+
+// The output tiles of a map: th rows x kTW columns, tile t = (t / tx, t % tx).
+struct Tiles {
+    int h, w, th, tx, n;
+    float inv_tx;
+    __device__ __forceinline__ int count(int t) const {  // pixels of tile t
+        const int ty = (int)(((float)t + 0.5f) * inv_tx);  // exact below 2^21 tiles
+        return min(th, h - ty * th) * min(kTW, w - (t - ty * tx) * kTW);
+    }
 };
 
 struct EncArgs {
@@ -66,28 +77,106 @@ struct EncArgs {
     float* net;  // kEpNetInp
     float* inp;
     long ni_nstride;
+    float2* stats;       // kEpStats: [image][tile][co_pad] (mean, sum of squared deviations)
+    // k_enc_conv<.., kDown>: the block's 1x1 downsampling beside this convolution
+    const _Float16* wt_d;
+    const float* bias_d;
+    _Float16* out_d;
+    float2* stats_d;
 };
+
+// (mean, 1/sqrt(var + 1e-5)) of NC channels c0 .. of image n into mom[NC], from
+// the statistics that the tiles of the convolution left ([image][tile][C]).
+// NC / 2 threads hold two channels each, so that a wave's loads are whole
+// rows; 512 / NC such groups share the tiles (12 loads in flight a thread) and
+// are added through LDS in order. All 256 threads take part; sums in double.
+// Contains a barrier, before mom is written.
+template <int NC>
+__device__ __forceinline__ void in_moments(const float2* part, int n, const Tiles& tl, int C,
+                                           int c0, float2* mom) {
+    constexpr int G = 512 / NC, NB = 12;
+    __shared__ double2 red[2][256];
+    const int t = threadIdx.x, c = t % (NC / 2), j = t / (NC / 2);
+    const float4* q = reinterpret_cast<const float4*>(part + (long)n * tl.n * C + c0) + c;
+    double2 s1 = {0.0, 0.0}, s2 = {0.0, 0.0};
+    const bool ragged = tl.h % tl.th != 0 || tl.w % kTW != 0;
+    for (int b = j; b < tl.n; b += NB * G) {
+        float4 v[NB];
+#pragma unroll
+        for (int u = 0; u < NB; u++) v[u] = q[(long)min(b + u * G, tl.n - 1) * (C / 2)];
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int s = b + u * G;
+            if (s < tl.n) {
+                const double cnt = ragged ? tl.count(s) : tl.th * kTW;
+                const double m0 = v[u].x, m1 = v[u].z, w0 = m0 * cnt, w1 = m1 * cnt;
+                s1.x += w0;
+                s1.y += w1;
+                s2.x += w0 * m0 + (double)v[u].y;
+                s2.y += w1 * m1 + (double)v[u].w;
+            }
+        }
+    }
+    red[0][t] = s1;
+    red[1][t] = s2;
+    __syncthreads();
+    if (t < NC) {
+        const double* r1 = reinterpret_cast<const double*>(red[0]) + t;
+        const double* r2 = reinterpret_cast<const double*>(red[1]) + t;
+        double a1 = 0.0, a2 = 0.0;
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            a1 += r1[g * NC];
+            a2 += r2[g * NC];
+        }
+        const double hw = (double)tl.h * tl.w, mean = a1 / hw, var = a2 / hw - mean * mean;
+        mom[t] = make_float2((float)mean, 1.0f / sqrtf((float)(var < 0.0 ? 0.0 : var) + 1e-5f));
+    }
+}
+
+// What a lane's epilogue reads, loaded at the kernel's start: the 16 biases of
+// its channels and, for kEpAddRelu, the residual (of a clamped pixel). Read in
+// the epilogue they were a trip to memory at the end of each launch.
+struct EpiLoads {
+    float4 bias[4];
+    f16x4 res[4];
+};
+template <int EPI>
+__device__ __forceinline__ EpiLoads epi_load(const float* bias, const EncArgs& a, int n, int co0,
+                                             int p, int ohw) {
+    EpiLoads e;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        e.bias[g] = *reinterpret_cast<const float4*>(bias + co0 + 8 * g);
+        if constexpr (EPI == kEpAddRelu) {
+            const int co = min(co0 + 8 * g, a.Co - 4);
+            e.res[g] = *reinterpret_cast<const f16x4*>(
+                a.res + (long)n * a.res_nstride + ((long)(co >> 4) * ohw + p) * 16 + (co & 15));
+        }
+    }
+    return e;
+}
 
 // The epilogue of one lane's accumulator block: register v holds output
 // channel co0 + 8*(v/4) + v%4 (co0 includes the lane's 4*lhi) at pixel p.
 template <int EPI>
-__device__ __forceinline__ void enc_epilogue(const EncArgs& a, const f32x16& acc, int n, int co0,
-                                             int p, int ohw) {
+__device__ __forceinline__ void enc_epilogue(const EncArgs& a, const f32x16& acc,
+                                             const EpiLoads& e, int n, int co0, int p, int ohw) {
 #pragma unroll
     for (int g = 0; g < 4; g++) {
         const int co = co0 + 8 * g;
         if (co >= a.Co) continue;
         float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = r16(r16(acc[4 * g + i]) + a.bias[co + i]);
+        for (int i = 0; i < 4; i++) v[i] = r16(r16(acc[4 * g + i]) + (&e.bias[g].x)[i]);
         const long ck = ((long)(co >> 4) * ohw + p) * 16 + (co & 15);
-        if constexpr (EPI == kEpRaw || EPI == kEpRelu) {
+        if constexpr (EPI == kEpRaw || EPI == kEpRelu || EPI == kEpStats) {
             f16x4 o;
 #pragma unroll
             for (int i = 0; i < 4; i++) o[i] = (_Float16)(EPI == kEpRelu ? fmaxf(v[i], 0.0f) : v[i]);
             *reinterpret_cast<f16x4*>(a.out + (long)n * a.out_nstride + ck) = o;
         } else if constexpr (EPI == kEpAddRelu) {
-            const f16x4 rs = *reinterpret_cast<const f16x4*>(a.res + (long)n * a.res_nstride + ck);
+            const f16x4 rs = e.res[g];
             f16x4 o;
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -110,17 +199,75 @@ __device__ __forceinline__ void enc_epilogue(const EncArgs& a, const f32x16& acc
     }
 }
 
+// kEpStats: mean and sum of squared deviations of the workgroup's tile per
+// channel (fp32, of the values as stored), into stats. Called by every
+// thread; `in`: the lane's pixel is in the map. A convolution's values are in
+// its registers here: a kernel of its own read them back, 4 us and a launch
+// after each of 15 convolutions of a frame.
+template <int WM>
+__device__ __forceinline__ void tile_stats(const EncArgs& a, const f32x16& acc,
+                                           const EpiLoads& e, float2* stats, int n,
+                                           int tile, int cot, int wm, int wn, bool in) {
+    constexpr int WN = 4 / WM, CO_T = WM * 32;
+    __shared__ float red[WN][CO_T], mean_s[CO_T];
+    const int tid = threadIdx.x, lane = tid & 63, lhi = lane >> 5;
+    const int ch0 = wm * 32 + 4 * lhi;  // register v: channel ch0 + 8 * (v / 4) + v % 4
+    float y[16], s[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        y[v] = in ? r16(r16(acc[v]) + (&e.bias[v / 4].x)[v % 4]) : 0.0f;
+        s[v] = y[v];
+    }
+    // the 32 lanes of a half wave: one channel's total a lane, then all rows
+    auto reduce = [&]() {
+        int base = 0, valid = 16;
+        rs_level<float, 16, 8>(s, lane, base, valid);
+        rs_level<float, 8, 4>(s, lane, base, valid);
+        rs_level<float, 4, 2>(s, lane, base, valid);
+        rs_level<float, 2, 1>(s, lane, base, valid);
+        s[0] += xchg<16>(s[0]);
+        if (!(lane & 16)) red[wn][ch0 + 8 * (base / 4) + base % 4] = s[0];
+        __syncthreads();
+        float r = 0.0f;
+        if (tid < CO_T) {
+            r = red[0][tid];
+#pragma unroll
+            for (int w = 1; w < WN; w++) r += red[w][tid];
+        }
+        return r;
+    };
+    const int th = min(WN, a.oh - tile / a.tiles_x * WN);
+    const float cnt = (float)(th * min(kTW, a.ow - tile % a.tiles_x * kTW));
+    const float mean = reduce() / cnt;
+    if (tid < CO_T) mean_s[tid] = mean;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        const float d = in ? y[v] - mean_s[ch0 + 8 * (v / 4) + v % 4] : 0.0f;
+        s[v] = d * d;
+    }
+    const float m2 = reduce();
+    if (tid < CO_T)
+        stats[((long)n * gridDim.y + tile) * a.co_pad + cot * CO_T + tid] = make_float2(mean, m2);
+}
+
 // 3x3 and 1x1 convolutions. One workgroup: 4 waves in a WM x WN grid, wave
 // (wm, wn) computing output channels cot*CO_T + wm*32 .. +31 of output row
 // ty0 + wn, 32 consecutive columns. The layers are small (at most 8 input
 // chunks, a few KB of patch per chunk), so a workgroup stages the input
 // patches of up to NCH chunks at once: every global load of the group is
 // issued before the first is stored to LDS, one barrier, then the MFMAs of
-// all NCH chunks. The weight fragments of chunk c+1 (all taps) are loaded
-// during chunk c's MFMAs (two register sets).
-template <int KS, int S, int WM, int NCH, int EPI>
-__global__ __launch_bounds__(256) void k_enc_conv(EncArgs a) {
-    static_assert(NCH % 2 == 0, "register sets alternate by chunk parity");
+// all NCH chunks. The weight fragments (all taps of a chunk) are loaded up to
+// three chunks ahead of their MFMAs, in up to four register sets (one chunk
+// ahead, a layer of 128 channels waited for each: 11.2 us, 9.6 so). The layers
+// of two chunks, which have the most tiles, keep two workgroups on a CU.
+// kDown: a block's 1x1 convolution of the same input and stride, on the patch's
+// centre taps, into an accumulator of its own (its launch took 5.4 us and, in
+// an encoder's chain, the gap before it).
+template <int KS, int S, int WM, int NCH, int EPI, bool kDown>
+__global__ __launch_bounds__(256, NCH < 4 ? 2 : 1) void k_enc_conv(EncArgs a) {
+    constexpr int SETS = NCH < 4 ? NCH : 4;
+    static_assert(NCH % SETS == 0, "register sets rotate by chunk");
     constexpr int WN = 4 / WM, TH = WN, CO_T = WM * 32;
     constexpr int P = KS / 2;
     constexpr int PH = S * (TH - 1) + KS, PW = S * (kTW - 1) + KS;
@@ -139,60 +286,93 @@ __global__ __launch_bounds__(256) void k_enc_conv(EncArgs a) {
 
     const _Float16* wbase = a.wt + ((long)cot * CO_T + wm * 32 + l32) * 16 + lhi * 8;
     const long tap_stride = (long)a.nchunk * a.co_pad * 16;
-    f16x8 A[2][TAPS];
+    f16x8 A[SETS][TAPS];
     auto load_a = [&](int c, f16x8* dst) {
 #pragma unroll
         for (int t = 0; t < TAPS; t++)
             dst[t] = *reinterpret_cast<const f16x8*>(wbase + t * tap_stride + (long)c * a.co_pad * 16);
     };
-    load_a(0, A[0]);
-    f32x16 acc = {};
+#pragma unroll
+    for (int q = 0; q < SETS - 1; q++)
+        if (q < a.nchunk) load_a(q, A[q]);
+    const int oy = ty0 + wn, ox = tx0 + l32, co0 = cot * CO_T + wm * 32 + 4 * lhi;
+    const EpiLoads el = epi_load<EPI>(a.bias, a, n, co0, min(oy, a.oh - 1) * a.ow + min(ox, a.ow - 1),
+                                      a.oh * a.ow);
+    const EpiLoads ed = kDown ? epi_load<EPI>(a.bias_d, a, n, co0, 0, 0) : EpiLoads{};
+    f16x8 D[NCH];  // kDown: all its weights (nchunk <= NCH)
+    if constexpr (kDown)
+#pragma unroll
+        for (int q = 0; q < NCH; q++)
+            D[q] = *reinterpret_cast<const f16x8*>(
+                a.wt_d + ((long)min(q, a.nchunk - 1) * a.co_pad + cot * CO_T + wm * 32 + l32) * 16 +
+                lhi * 8);
+    f32x16 acc = {}, accd = {};
     for (int g0 = 0; g0 < a.nchunk; g0 += NCH) {
         const int ng = min(NCH, a.nchunk - g0);
         if (g0 > 0) __syncthreads();  // the previous group's patches are consumed
+        // every load unconditional, from a clamped chunk and pixel
         f16x8 reg[NCH][UPT];
+        bool ok[UPT];
+        int off[UPT];
 #pragma unroll
-        for (int q = 0; q < NCH; q++) {
-            const _Float16* base = a.in + (long)n * a.in_nstride + (long)(g0 + q) * ihw * 16;
-#pragma unroll
-            for (int u = 0; u < UPT; u++) {
-                const int unit = tid + 256 * u;
-                const int pix = unit >> 1, half = unit & 1;
-                const int py = pix / PW, px = pix - (pix / PW) * PW;
-                const int y = iy0 + py, x = ix0 + px;
-                const bool ok = q < ng && unit < UNITS && y >= 0 && y < a.ih && x >= 0 && x < a.iw;
-                f16x8 v = {};
-                if (ok) v = *reinterpret_cast<const f16x8*>(base + ((long)y * a.iw + x) * 16 + half * 8);
-                reg[q][u] = v;
-            }
+        for (int u = 0; u < UPT; u++) {
+            const int unit = tid + 256 * u;
+            const int pix = min(unit, UNITS - 1) >> 1, half = unit & 1;
+            const int py = pix / PW, px = pix - (pix / PW) * PW;
+            const int y = iy0 + py, x = ix0 + px;
+            ok[u] = y >= 0 && y < a.ih && x >= 0 && x < a.iw;
+            off[u] = (min(max(y, 0), a.ih - 1) * a.iw + min(max(x, 0), a.iw - 1)) * 16 + half * 8;
         }
 #pragma unroll
-        for (int q = 0; q < NCH; q++)
+        for (int q = 0; q < NCH; q++) {
+            const _Float16* base =
+                a.in + (long)n * a.in_nstride + (long)(g0 + min(q, ng - 1)) * ihw * 16;
 #pragma unroll
-            for (int u = 0; u < UPT; u++) {
-                const int unit = tid + 256 * u;
-                if (q < ng && unit < UNITS) *reinterpret_cast<f16x8*>(&patch[q][unit * 8]) = reg[q][u];
+            for (int u = 0; u < UPT; u++) reg[q][u] = *reinterpret_cast<const f16x8*>(base + off[u]);
+        }
+#pragma unroll
+        for (int q = 0; q < NCH; q++) {
+            if (q < ng) {
+#pragma unroll
+                for (int u = 0; u < UPT; u++) {
+                    const int unit = tid + 256 * u;
+                    if (unit < UNITS)
+                        *reinterpret_cast<f16x8*>(&patch[q][unit * 8]) = ok[u] ? reg[q][u] : f16x8{};
+                }
             }
+        }
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < NCH; q++) {
             if (q < ng) {
                 const int c = g0 + q;
-                if (c + 1 < a.nchunk) load_a(c + 1, A[(q + 1) & 1]);
+                if (c + SETS - 1 < a.nchunk) load_a(c + SETS - 1, A[(q + SETS - 1) % SETS]);
                 const _Float16* pb = &patch[q][0];
 #pragma unroll
                 for (int t = 0; t < TAPS; t++) {
                     const int ky = t / KS, kx = t - (t / KS) * KS;
                     const f16x8 b = *reinterpret_cast<const f16x8*>(
                         pb + (((S * wn + ky) * PW + S * l32 + kx) * 16 + lhi * 8));
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[q & 1][t], b, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[q % SETS][t], b, acc, 0, 0, 0);
+                    if constexpr (kDown)
+                        if (t == TAPS / 2)
+                            accd = __builtin_amdgcn_mfma_f32_32x32x16_f16(D[q], b, accd, 0, 0, 0);
                 }
             }
         }
     }
-    const int y = ty0 + wn, x = tx0 + l32;
-    if (y < a.oh && x < a.ow)
-        enc_epilogue<EPI>(a, acc, n, cot * CO_T + wm * 32 + 4 * lhi, y * a.ow + x, a.oh * a.ow);
+    const bool in = oy < a.oh && ox < a.ow;
+    if (in) enc_epilogue<EPI>(a, acc, el, n, co0, oy * a.ow + ox, a.oh * a.ow);
+    if constexpr (EPI == kEpStats) tile_stats<WM>(a, acc, el, a.stats, n, tile, cot, wm, wn, in);
+    if constexpr (kDown) {
+        a.out = a.out_d;
+        constexpr int ED = EPI == kEpStats ? kEpStats : kEpRaw;
+        if (in) enc_epilogue<ED>(a, accd, ed, n, co0, oy * a.ow + ox, a.oh * a.ow);
+        if constexpr (EPI == kEpStats) {
+            __syncthreads();  // tile_stats' LDS is read
+            tile_stats<WM>(a, accd, ed, a.stats_d, n, tile, cot, wm, wn, in);
+        }
+    }
 }
 
 // conv1 (7x7, stride 2, 3 -> 32 channels) with the taps packed into K: the
@@ -221,11 +401,14 @@ __global__ __launch_bounds__(256) void k_enc_stem(EncArgs a) {
         const int pix = tid + 256 * u;
         const int py = pix / PW, px = pix - (pix / PW) * PW;
         const int y = iy0 + py, x = ix0 + px;
-        f16x4 v = {};
-        if (pix < UNITS && y >= 0 && y < a.ih && x >= 0 && x < a.iw)
-            v = *reinterpret_cast<const f16x4*>(img + ((long)y * a.iw + x) * 4);
-        reg[u] = v;
+        // unconditional, from the nearest pixel
+        const f16x4 v = *reinterpret_cast<const f16x4*>(
+            img + ((long)min(max(y, 0), a.ih - 1) * a.iw + min(max(x, 0), a.iw - 1)) * 4);
+        reg[u] = y >= 0 && y < a.ih && x >= 0 && x < a.iw ? v : f16x4{};
     }
+    const int oy = ty0 + wn, ox = tx0 + l32;
+    const bool in = oy < a.oh && ox < a.ow;
+    const EpiLoads el = epi_load<EPI>(a.bias, a, n, 4 * lhi, 0, a.oh * a.ow);
     f16x8 A[KSTEPS];
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++)
@@ -248,105 +431,8 @@ __global__ __launch_bounds__(256) void k_enc_stem(EncArgs a) {
         const f16x8 b = {b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
         acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[ks], b, acc, 0, 0, 0);
     }
-    const int y = ty0 + wn, x = tx0 + l32;
-    if (y < a.oh && x < a.ow) enc_epilogue<EPI>(a, acc, n, 4 * lhi, y * a.ow + x, a.oh * a.ow);
-}
-
-constexpr int kSplit = 256;  // pixels per statistics split (2 per thread pair)
-
-// Per-split statistics of one 16-channel chunk of a CK tensor: pixels
-// [s*kSplit, min(hw, (s+1)*kSplit)) of image n; part[(n*nsplit + s)*C + c] =
-// (mean, sum of squared deviations from that mean), both in fp32. Thread t
-// holds channels 8*(t&1) .. +7 of pixels s*kSplit + (t>>1) + 128*i.
-__global__ __launch_bounds__(256) void k_in_stats(const _Float16* y, long nstride, int hw,
-                                                  int C, int nsplit, float2* part) {
-    __shared__ float red[4][2][8];
-    __shared__ float tot_s[16], mean_s[16], m2_s[16];
-    const int ch = blockIdx.x, s = blockIdx.y, n = blockIdx.z;
-    const int t = threadIdx.x, half = t & 1, pl = t >> 1;
-    const int lane = t & 63, wave = t >> 6;
-    const int p0 = s * kSplit, p1 = min(hw, p0 + kSplit);
-    const _Float16* base = y + (long)n * nstride + (long)ch * hw * 16 + half * 8;
-    constexpr int kIt = kSplit / 128;
-    f16x8 v[kIt];
-    float acc[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) acc[k] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kIt; i++) {
-        const int p = p0 + pl + 128 * i;
-        v[i] = f16x8{};
-        if (p < p1) v[i] = *reinterpret_cast<const f16x8*>(base + (long)p * 16);
-#pragma unroll
-        for (int k = 0; k < 8; k++) acc[k] += (float)v[i][k];
-    }
-    // sum over the 128 threads of one half: lanes of equal parity, then waves
-    auto reduce = [&](float* vals, float* outv) {
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            float x = vals[k];
-#pragma unroll
-            for (int off = 2; off < 64; off <<= 1) x += __shfl_xor(x, off);
-            vals[k] = x;
-        }
-        if (lane < 2) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) red[wave][lane][k] = vals[k];
-        }
-        __syncthreads();
-        if (t < 16) {
-            const int hh = t >> 3, k = t & 7;
-            outv[t] = ((red[0][hh][k] + red[1][hh][k]) + red[2][hh][k]) + red[3][hh][k];
-        }
-        __syncthreads();
-    };
-    reduce(acc, tot_s);
-    const float cnt = (float)(p1 - p0);
-    if (t < 16) mean_s[t] = tot_s[t] / cnt;
-    __syncthreads();
-    float m[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) m[k] = mean_s[half * 8 + k];
-#pragma unroll
-    for (int k = 0; k < 8; k++) acc[k] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kIt; i++) {
-        if (p0 + pl + 128 * i < p1) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const float d = (float)v[i][k] - m[k];
-                acc[k] += d * d;
-            }
-        }
-    }
-    reduce(acc, m2_s);
-    if (t < 16) part[((long)n * nsplit + s) * C + ch * 16 + t] = make_float2(mean_s[t], m2_s[t]);
-}
-
-// (mean, 1/sqrt(var + 1e-5)) of the 16 channels of chunk ch of image n from
-// their nsplit partials, into mom[16]: 16 threads per channel (all 256 of
-// the workgroup take part), the total mean from the count-weighted split
-// means, then the sum of squared deviations as sum_s M2_s + n_s (mean_s -
-// mean)^2, each a fixed-order sum per thread and a fixed butterfly over
-// the 16 threads.
-__device__ void in_moments16(const float2* part, int n, int nsplit, int C, int ch, int hw,
-                             float2* mom) {
-    const int t = threadIdx.x, c = t >> 4, j = t & 15;
-    const float2* q = part + (long)n * nsplit * C + ch * 16 + c;
-    float s1 = 0.0f;
-    for (int s = j; s < nsplit; s += 16) s1 += (float)min(kSplit, hw - s * kSplit) * q[(long)s * C].x;
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) s1 += __shfl_xor(s1, off);
-    const float mean = s1 / (float)hw;
-    float s2 = 0.0f;
-    for (int s = j; s < nsplit; s += 16) {
-        const float2 v = q[(long)s * C];
-        const float d = v.x - mean;
-        s2 += v.y + (float)min(kSplit, hw - s * kSplit) * d * d;
-    }
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) s2 += __shfl_xor(s2, off);
-    if (j == 0) mom[c] = make_float2(mean, 1.0f / sqrtf(s2 / (float)hw + 1e-5f));
+    if (in) enc_epilogue<EPI>(a, acc, el, n, 4 * lhi, oy * a.ow + ox, a.oh * a.ow);
+    if constexpr (EPI == kEpStats) tile_stats<1>(a, acc, el, a.stats, n, tile, 0, 0, wn, in);
 }
 
 enum InMode {
@@ -356,41 +442,55 @@ enum InMode {
 };
 
 // Normalises one CK tensor in place (or into out), fused with the block's
-// ReLU and residual add: grid (ceil(hw/128), C/16, images), thread = 8
-// channels of one pixel.
-template <int MODE>
+// ReLU and residual add: grid (ceil(hw/(128 R)), C/16, images), thread = 8
+// channels of R pixels. Bound by two trips to memory, pixels and statistics
+// together and then the store: 5.1 us for 32 channels of 192x256 (7.6 us with
+// the statistics read one by one).
+template <int MODE, int R>
 __global__ __launch_bounds__(256) void k_in_apply(_Float16* y, const float2* part,
                                                   const _Float16* res, const float2* part2,
                                                   _Float16* out, long nstride, int hw, int C,
-                                                  int nsplit) {
+                                                  Tiles tl) {
     __shared__ float2 mom[2][16];
     const int ch = blockIdx.y, n = blockIdx.z, t = threadIdx.x;
-    in_moments16(part, n, nsplit, C, ch, hw, mom[0]);
-    if constexpr (MODE == kInAddNorm) in_moments16(part2, n, nsplit, C, ch, hw, mom[1]);
-    __syncthreads();
-    const int p = blockIdx.x * 128 + (t >> 1), half = t & 1;
-    if (p >= hw) return;
-    const long off = (long)n * nstride + ((long)ch * hw + p) * 16 + half * 8;
-    const f16x8 v = *reinterpret_cast<const f16x8*>(y + off);
-    f16x8 rs = {};
-    if constexpr (MODE != kInRelu) rs = *reinterpret_cast<const f16x8*>(res + off);
-    f16x8 o;
+    // the pixels' own loads first, under the moments' (a pixel past the map
+    // reads the last one and stores nothing)
+    const int p0 = blockIdx.x * (128 * R) + (t >> 1), half = t & 1;
+    const long base = (long)n * nstride + (long)ch * hw * 16 + half * 8;
+    f16x8 v[R], rs[R];
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const float2 m = mom[0][half * 8 + k];
-        const float nv = fmaxf(r16(((float)v[k] - m.x) * m.y), 0.0f);
-        if constexpr (MODE == kInRelu) {
-            o[k] = (_Float16)nv;
-        } else {
-            float r = (float)rs[k];
-            if constexpr (MODE == kInAddNorm) {
-                const float2 m2 = mom[1][half * 8 + k];
-                r = r16((r - m2.x) * m2.y);
-            }
-            o[k] = (_Float16)fmaxf(r16(nv + r), 0.0f);
-        }
+    for (int r = 0; r < R; r++) {
+        const long off = base + (long)min(p0 + 128 * r, hw - 1) * 16;
+        v[r] = *reinterpret_cast<const f16x8*>(y + off);
+        if constexpr (MODE != kInRelu) rs[r] = *reinterpret_cast<const f16x8*>(res + off);
     }
-    *reinterpret_cast<f16x8*>((MODE == kInRelu ? y : out) + off) = o;
+    in_moments<16>(part, n, tl, C, ch * 16, mom[0]);
+    if constexpr (MODE == kInAddNorm) {
+        __syncthreads();  // in_moments' LDS is read
+        in_moments<16>(part2, n, tl, C, ch * 16, mom[1]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int p = p0 + 128 * r;
+        f16x8 o;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float2 m = mom[0][half * 8 + k];
+            const float nv = fmaxf(r16(((float)v[r][k] - m.x) * m.y), 0.0f);
+            if constexpr (MODE == kInRelu) {
+                o[k] = (_Float16)nv;
+            } else {
+                float x = (float)rs[r][k];
+                if constexpr (MODE == kInAddNorm) {
+                    const float2 m2 = mom[1][half * 8 + k];
+                    x = r16((x - m2.x) * m2.y);
+                }
+                o[k] = (_Float16)fmaxf(r16(nv + x), 0.0f);
+            }
+        }
+        if (p < hw) *reinterpret_cast<f16x8*>((MODE == kInRelu ? y : out) + base + (long)p * 16) = o;
+    }
 }
 
 // The encoder input as [image][h*w][4] fp16 (R, G, B, 0). From the caller's BGR frame (H x W x 3,
@@ -417,6 +517,12 @@ __global__ void k_image_to_px4(const float* src, int from_bgr, long src_nstride,
 }
 
 // ---------------------------------------------------------------- host side
+// k_in_apply takes the widest tile that gives this many workgroups: each reads
+// the statistics of all tiles (49 KB at the first stage of a 384x512 image), so
+// few wide ones read them less often. The seven ReLU launches of that image: 35
+// us at R = 1 throughout, 33.5 at R = 4, 32 so (4, 2, 1 by stage).
+constexpr long kApplyWgs = 192;
+
 constexpr int kEncLayers = 16;
 struct EncLayer {
     const char* suffix;
@@ -449,7 +555,7 @@ struct slk_encoder_state {
     bool have[kEncLayers] = {};
     bool packed = false;
     EncPacked pk[kEncLayers];
-    DevBuf img, A, B, T, D, part1, part2;
+    DevBuf img, A, B, T, D, part[2];
     // encode_frame runs the context encoder on this stream (non-blocking,
     // default priority) beside the feature encoder on the caller's, forked
     // and joined by the two events; created on the first such call
@@ -517,14 +623,28 @@ struct Act {
 };
 Act ck_act(_Float16* p, int nch, int h, int w) { return Act{p, nch, h, w, (long)nch * h * w * 16}; }
 
+// the output tiles of an h x w map of C channels (32 channels x 4 rows, 64 x 2
+// or 128 x 1, x kTW columns)
+Tiles tiles_of(int C, int h, int w) {
+    const int th = 128 / co_tile(C), tx = (w + kTW - 1) / kTW;
+    return Tiles{h, w, th, tx, tx * ((h + th - 1) / th), 1.0f / (float)tx};
+}
+
 template <int KS, int S, int WM, int NCH, int EPI>
 void launch_cfg(const EncArgs& a, int N, hipStream_t stream) {
     constexpr int TH = 4 / WM, CO_T = WM * 32;
     const int tiles_y = (a.oh + TH - 1) / TH;
     EncArgs b = a;
     b.tiles_x = (a.ow + kTW - 1) / kTW;
-    hipLaunchKernelGGL((k_enc_conv<KS, S, WM, NCH, EPI>), dim3(a.co_pad / CO_T, b.tiles_x * tiles_y, N),
-                       dim3(256), 0, stream, b);
+    const dim3 grid(a.co_pad / CO_T, b.tiles_x * tiles_y, N);
+    if constexpr (KS == 3 && S == 2 && (EPI == kEpStats || EPI == kEpRelu)) {
+        if (a.wt_d) {  // nchunk == NCH for both layers of this shape
+            hipLaunchKernelGGL((k_enc_conv<KS, S, WM, NCH, EPI, true>), grid, dim3(256), 0, stream,
+                               b);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_enc_conv<KS, S, WM, NCH, EPI, false>), grid, dim3(256), 0, stream, b);
 }
 
 template <int EPI>
@@ -546,22 +666,30 @@ int launch_layer(const EncPacked& pc, EncArgs a, int N, hipStream_t stream) {
     } else if (cot == 32 && pc.k == 3 && pc.s == 1) launch_cfg<3, 1, 1, 2, EPI>(a, N, stream);
     else if (cot == 64 && pc.k == 3 && pc.s == 2) launch_cfg<3, 2, 2, 2, EPI>(a, N, stream);
     else if (cot == 64 && pc.k == 3 && pc.s == 1) launch_cfg<3, 1, 2, 4, EPI>(a, N, stream);
-    else if (cot == 64 && pc.k == 1 && pc.s == 2) launch_cfg<1, 2, 2, 2, EPI>(a, N, stream);
     else if (cot == 128 && pc.k == 3 && pc.s == 2) launch_cfg<3, 2, 4, 4, EPI>(a, N, stream);
     else if (cot == 128 && pc.k == 3 && pc.s == 1) launch_cfg<3, 1, 4, 8, EPI>(a, N, stream);
-    else if (cot == 128 && pc.k == 1 && pc.s == 2) launch_cfg<1, 2, 4, 4, EPI>(a, N, stream);
     else if (cot == 128 && pc.k == 1 && pc.s == 1) launch_cfg<1, 1, 4, 8, EPI>(a, N, stream);
     else return fail(SLK_E_ARG, "encoder: no kernel for this layer shape");
     SLK_HIP(hipGetLastError());
     return SLK_OK;
 }
 
-// conv of layer L from x into a new activation at `dst`
+// conv of layer L from x into a new activation at `dst`; kEpStats leaves its
+// statistics in `stats`; with down, the block's downsampling of x (layer L + 2)
+// to `down` as well
 template <int EPI>
 int conv(const slk_encoder_state& e, int L, const Act& x, _Float16* dst, Act* y, int N,
-         hipStream_t stream, const Act* res = nullptr) {
+         hipStream_t stream, const Act* res = nullptr, float2* stats = nullptr,
+         _Float16* down = nullptr, float2* stats_d = nullptr) {
     const EncPacked& pc = e.pk[L];
     EncArgs a{};
+    a.stats = stats;
+    if (down) {
+        a.wt_d = e.pk[L + 2].wt.as<_Float16>();
+        a.bias_d = e.pk[L + 2].bias.as<float>();
+        a.out_d = down;
+        a.stats_d = stats_d;
+    }
     a.in = x.p;
     a.in_nstride = x.ns;
     a.ih = x.h;
@@ -578,21 +706,22 @@ int conv(const slk_encoder_state& e, int L, const Act& x, _Float16* dst, Act* y,
     return launch_layer<EPI>(pc, a, N, stream);
 }
 
-int nsplit_of(int hw) { return (hw + kSplit - 1) / kSplit; }
-
-void in_stats(const Act& y, float2* part, int N, hipStream_t stream) {
+template <int MODE, int R>
+void launch_apply(const Act& y, const float2* part, const Act* res, const float2* part2,
+                  _Float16* out, int N, hipStream_t stream) {
     const int hw = y.h * y.w;
-    hipLaunchKernelGGL(k_in_stats, dim3(y.nch, nsplit_of(hw), N), dim3(256), 0, stream, y.p,
-                       y.ns, hw, y.nch * 16, nsplit_of(hw), part);
+    hipLaunchKernelGGL((k_in_apply<MODE, R>), dim3((hw + 128 * R - 1) / (128 * R), y.nch, N),
+                       dim3(256), 0, stream, y.p, part, res ? res->p : nullptr, part2, out, y.ns,
+                       hw, y.nch * 16, tiles_of(y.nch * 16, y.h, y.w));
 }
 
 template <int MODE>
 void in_apply(const Act& y, const float2* part, const Act* res, const float2* part2, _Float16* out,
               int N, hipStream_t stream) {
-    const int hw = y.h * y.w;
-    hipLaunchKernelGGL((k_in_apply<MODE>), dim3((hw + 127) / 128, y.nch, N), dim3(256), 0, stream,
-                       y.p, part, res ? res->p : nullptr, part2, out, y.ns, hw, y.nch * 16,
-                       nsplit_of(hw));
+    const long wgs = (long)(y.h * y.w + 511) / 512 * y.nch * N;  // at R = 4
+    if (wgs >= kApplyWgs) launch_apply<MODE, 4>(y, part, res, part2, out, N, stream);
+    else if (2 * wgs >= kApplyWgs) launch_apply<MODE, 2>(y, part, res, part2, out, N, stream);
+    else launch_apply<MODE, 1>(y, part, res, part2, out, N, stream);
 }
 
 // HalfBasicEncoder::forward from a CK image to the last layer,
@@ -600,17 +729,16 @@ void in_apply(const Act& y, const float2* part, const Act* res, const float2* pa
 template <typename Finish>
 int encoder_run(slk_encoder_state& e, const _Float16* image, int N, hipStream_t stream,
                 Finish finish) {
-    float2* p1 = e.part1.as<float2>();
-    float2* p2 = e.part2.as<float2>();
+    float2* py = e.part[0].as<float2>();  // statistics of the last convolution
+    float2* pd = e.part[1].as<float2>();  // and of a block's downsampling
     Act img{const_cast<_Float16*>(image), 1, e.in_h, e.in_w, 4L * e.in_h * e.in_w};
     Act x, y, t, d;
     _Float16* bufA = e.A.as<_Float16>();
     _Float16* bufB = e.B.as<_Float16>();
     // conv1 (7x7, stride 2) + norm + relu (main.cu:363-365)
     if (e.norm) {
-        SLK_TRY(conv<kEpRaw>(e, 0, img, bufA, &x, N, stream));
-        in_stats(x, p1, N, stream);
-        in_apply<kInRelu>(x, p1, nullptr, nullptr, nullptr, N, stream);
+        SLK_TRY(conv<kEpStats>(e, 0, img, bufA, &x, N, stream, nullptr, py));
+        in_apply<kInRelu>(x, py, nullptr, nullptr, nullptr, N, stream);
     } else {
         SLK_TRY(conv<kEpRelu>(e, 0, img, bufA, &x, N, stream));
     }
@@ -619,23 +747,20 @@ int encoder_run(slk_encoder_state& e, const _Float16* image, int N, hipStream_t 
         const int c1 = blk == 0 ? 1 : blk == 1 ? 3 : blk == 2 ? 5 : blk == 3 ? 8 : blk == 4 ? 10 : 13;
         const bool ds = blk == 2 || blk == 4;
         _Float16* out = x.p == bufA ? bufB : bufA;
+        _Float16* down = ds ? e.D.as<_Float16>() : nullptr;
         if (e.norm) {
-            SLK_TRY(conv<kEpRaw>(e, c1, x, e.T.as<_Float16>(), &t, N, stream));
-            in_stats(t, p1, N, stream);
-            in_apply<kInRelu>(t, p1, nullptr, nullptr, nullptr, N, stream);
+            SLK_TRY(conv<kEpStats>(e, c1, x, e.T.as<_Float16>(), &t, N, stream, nullptr, py, down, pd));
+            in_apply<kInRelu>(t, py, nullptr, nullptr, nullptr, N, stream);
+            SLK_TRY(conv<kEpStats>(e, c1 + 1, t, out, &y, N, stream, nullptr, py));
             if (ds) {
-                SLK_TRY(conv<kEpRaw>(e, c1 + 2, x, e.D.as<_Float16>(), &d, N, stream));
-                in_stats(d, p2, N, stream);
+                d = ck_act(down, y.nch, y.h, y.w);
+                in_apply<kInAddNorm>(y, py, &d, pd, out, N, stream);
+            } else {
+                in_apply<kInAddRelu>(y, py, &x, nullptr, out, N, stream);
             }
-            SLK_TRY(conv<kEpRaw>(e, c1 + 1, t, out, &y, N, stream));
-            in_stats(y, p1, N, stream);
-            if (ds)
-                in_apply<kInAddNorm>(y, p1, &d, p2, out, N, stream);
-            else
-                in_apply<kInAddRelu>(y, p1, &x, nullptr, out, N, stream);
         } else {
-            SLK_TRY(conv<kEpRelu>(e, c1, x, e.T.as<_Float16>(), &t, N, stream));
-            if (ds) SLK_TRY(conv<kEpRaw>(e, c1 + 2, x, e.D.as<_Float16>(), &d, N, stream));
+            SLK_TRY(conv<kEpRelu>(e, c1, x, e.T.as<_Float16>(), &t, N, stream, nullptr, nullptr, down));
+            if (ds) d = ck_act(down, t.nch, t.h, t.w);
             SLK_TRY(conv<kEpAddRelu>(e, c1 + 1, t, out, &y, N, stream, ds ? &d : &x));
         }
         SLK_HIP(hipGetLastError());
@@ -681,12 +806,14 @@ extern "C" int slk_encoder_create(slk_encoder** out, int in_h, int in_w, int out
     // the largest activation: 32 channels at half resolution (= 64 at a
     // quarter, 128 at an eighth)
     const size_t act = N * 32 * h2 * sizeof(_Float16);
-    const size_t parts = N * (size_t)nsplit_of((int)h2) * 128 * sizeof(float2);
+    size_t parts = 0;  // statistics of the stage with the most
+    for (int k = 1; k <= 3; k++)
+        parts = std::max(parts, N * tiles_of(16 << k, in_h >> k, in_w >> k).n * (16 << k) * sizeof(float2));
     int st = e.img.ensure(N * hw * 4 * sizeof(_Float16));
     for (DevBuf* b : {&e.A, &e.B, &e.T, &e.D})
         if (st == SLK_OK) st = b->ensure(act);
-    if (st == SLK_OK) st = e.part1.ensure(parts);
-    if (st == SLK_OK) st = e.part2.ensure(parts);
+    for (DevBuf& b : e.part)
+        if (st == SLK_OK && use_norm) st = b.ensure(parts);
     if (st != SLK_OK) {
         slk_encoder_destroy(enc);
         return st;
@@ -702,7 +829,8 @@ extern "C" int slk_encoder_destroy(slk_encoder* enc) {
         pc.wt.release();
         pc.bias.release();
     }
-    for (DevBuf* b : {&e.img, &e.A, &e.B, &e.T, &e.D, &e.part1, &e.part2}) b->release();
+    for (DevBuf* b : {&e.img, &e.A, &e.B, &e.T, &e.D}) b->release();
+    for (DevBuf& b : e.part) b.release();
     if (e.side) {
         // the side stream's work is finished before its resources go
         (void)hipStreamSynchronize(e.side);

@@ -65,6 +65,28 @@ def test_encoder_forward_batch(slk, prefix, out_dim, norm):
     check(got, ref, f"{prefix} 64x96")
 
 
+@pytest.mark.parametrize("h,w,n", [(40, 264, 1), (72, 136, 3), (16, 12400, 1)])
+@pytest.mark.parametrize("prefix,out_dim,norm", [("fnet", 128, True), ("cnet", 256, False)])
+def test_encoder_tile_edges(slk, prefix, out_dim, norm, h, w, n):
+    """Instance norms from the convolutions' tiles: tiles cut by both borders
+    at every stage (rows of 4, 2 and 1, columns of 32), several images, and
+    more tiles (388) than one batch of a normalising thread's loads (384). The
+    statistics are fp32 of at most 128 values, combined in double; the file's
+    bar holds."""
+    announce(f"encoder {prefix} {n} x {h}x{w}")
+    P = eo.seeded_weights(prefix, out_dim, seed=52)
+    img = np.random.default_rng(53).standard_normal((n, 3, h, w)).astype(np.float32)
+    enc = slk.Encoder(h, w, out_dim, norm, max_batch=n)
+    enc.set_weights(P, prefix)
+    d_in = slk.DeviceArray.from_host(img)
+    d_out = slk.DeviceArray((n, out_dim, h // 8, w // 8), np.float16)
+    enc.forward(d_in, d_out, batch=n)
+    slk.hip().sync()
+    got = d_out.to_host().astype(np.float64)
+    enc.close()
+    check(got, eo.encoder(uo.round16(img), P, prefix, norm), f"{prefix} {n}x{h}x{w}")
+
+
 def test_encode_frame_full_size(slk):
     """encode_frame on a 384 x 512 BGR frame (the 48 x 64 feature maps of
     the headline window): fmap fp16, net = tanh, inp = relu."""
