@@ -19,7 +19,7 @@
 //                 to the four blocks with the edge's Adj.
 //   k_ba_schur    [E; w] Q [E; w]^T per keyframe on fp64 MFMA: the blocks of
 //                 its pairs of E rows and E_r Q w per row.
-//   k_ba_assemble one workgroup per 6x6 block of S and per 6 entries of b:
+//   k_ba_assemble one workgroup per non-empty 6x6 block of S and per 6 entries of b:
 //                 sums the totals listed for the block (lists built on the
 //                 host; fixed order, no atomics), then S_ii += ep + lm*S_ii.
 //   k_ba_solve_*  fp64 factorization and solve, dx rounded to fp32,
@@ -671,34 +671,70 @@ struct SolveArgs {
                         // before the retraction (the overlapped step's ready flag)
 };
 
-// an entry of stot: its pixel shares in order
-__device__ __forceinline__ double stot_sum(const SolveArgs& A, size_t i) {
-    double t = A.stot[i];
-    for (int k = 1; k < A.nsp; k++) t += A.stot[k * A.share + i];
-    return t;
-}
-
-// One edge-block or Schur-item contribution to entry (r, c) of a 6x6 block of
-// S (ba.cuh:520-548, 722-742): code cd of the block's contribution list.
-__device__ __forceinline__ double s_contrib(const SolveArgs& A, int cd, int r, int c) {
+// Where an entry (r, c) of a contribution to a 6x6 block of S lies (edge block
+// or Schur item, ba.cuh:520-548, 722-742; code cd of the block's list): one
+// total of an edge, or n pixel shares to be added in order and subtracted.
+struct Contrib {
+    const double* p;
+    int n;
+    bool neg;
+};
+__device__ __forceinline__ Contrib s_contrib(const SolveArgs& A, int cd, int r, int c) {
     const int ty = code_type(cd), v = code_val(cd);
     if (ty == 0) {
         const double* et = A.etot + (size_t)(v >> 2) * kNT;
         const int w = v & 3;
-        return w == 0 ? et[kTotHii + r * 6 + c]
-             : w == 1 ? et[kTotHij + r * 6 + c]
-             : w == 2 ? et[kTotHij + c * 6 + r]
-                      : et[kTotHjj + r * 6 + c];
+        return {et + (w == 0   ? kTotHii + r * 6 + c
+                      : w == 1 ? kTotHij + r * 6 + c
+                      : w == 2 ? kTotHij + c * 6 + r
+                               : kTotHjj + r * 6 + c),
+                1, false};
     }
-    return -stot_sum(A, (size_t)v * 36 + (ty == 1 ? r * 6 + c : c * 6 + r));
+    return {A.stot + (size_t)v * 36 + (ty == 1 ? r * 6 + c : c * 6 + r), A.nsp, true};
 }
 
-// One workgroup per 6x6 block (a, b) of S (P*P of them) and per 6-entry
-// segment of b (P more): S = sum of the listed edge blocks minus the Schur
-// pair blocks, then the LM damping S_ii += ep + lm*S_ii after the Schur step
-// (ba.cuh:749-750); b = the edges' gradients minus E Q w of the pose's rows.
-// Thread (slice, entry) sums contributions slice, slice + 7, ... of the list,
-// and the seven slices are added in a fixed order (deterministic, no atomics).
+// The contributions q0, q0 + step, ... < q1 of `at`, added in that order; two
+// contributions of four shares each are in flight.
+template <typename At>
+__device__ __forceinline__ double sum_contribs(const SolveArgs& A, int q0, int q1,
+                                               int step, const At& at) {
+    constexpr int NC = 2;
+    double s = 0.0;
+    for (int q = q0; q < q1; q += NC * step) {
+        Contrib c[NC];
+        double v[NC][4];
+#pragma unroll
+        for (int u = 0; u < NC; u++) c[u] = at(q + u * step < q1 ? q + u * step : q);
+#pragma unroll
+        for (int u = 0; u < NC; u++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[u][k] = c[u].p[(size_t)min(k, c[u].n - 1) * A.share];
+#pragma unroll
+        for (int u = 0; u < NC; u++) {
+            if (q + u * step >= q1) continue;
+            double t = v[u][0];
+#pragma unroll
+            for (int k = 1; k < 4; k++)
+                if (k < c[u].n) t += v[u][k];
+            for (int k = 4; k < c[u].n; k++) t += c[u].p[(size_t)k * A.share];
+            s += c[u].neg ? -t : t;
+        }
+    }
+    return s;
+}
+
+// One workgroup per non-empty 6x6 block of S (n_blk of them; block (b, a) has the
+// transposes of (a, b)'s contributions in the same order, so the upper one's
+// workgroup writes both), per 6-entry segment of b (P more) and per row of blocks
+// (P more, the zeros of its empty ones): S =
+// sum of the listed edge blocks minus the Schur pair blocks, then the LM damping
+// S_ii += ep + lm*S_ii after the Schur step (ba.cuh:749-750); b = the edges'
+// gradients minus E Q w of the pose's rows. Thread (slice, entry) sums
+// contributions slice, slice + 7, ... of the list, and the seven slices are added
+// in a fixed order (deterministic, no atomics). Bound by the chain of loads (list
+// bounds, codes, entries) times the workgroups that a unit runs in turn: P = 198
+// with a workgroup for each of the P * P blocks, most of them empty, and one load
+// at a time took 43 us, 24 us so.
 constexpr int kAsmSlices = 7;  // 7 x 36 = 252 of the 256 threads
 __global__ __launch_bounds__(256) void k_ba_assemble(SolveArgs A) {
     __shared__ double red[kAsmSlices][36];
@@ -706,17 +742,14 @@ __global__ __launch_bounds__(256) void k_ba_assemble(SolveArgs A) {
     const int tid = threadIdx.x;
     const int sl = tid / 36, e = tid - sl * 36;
     const int g = blockIdx.x;
-    double s = 0.0;
-    if (g < P * P) {
-        const int a = g / P, bb = g - a * P;
+    if (g < A.n_blk) {
+        const int ab = A.plan.sblk[g], a = ab / P, bb = ab - a * P;
+        if (a > bb) return;  // the transpose's workgroup writes both
         const int r = e / 6, c = e - r * 6;
-        const int blk = A.plan.blkmap[g];
-        if (sl < kAsmSlices && blk >= 0) {
-            const int q1 = A.plan.sblk_ptr[blk + 1];
-            for (int q = A.plan.sblk_ptr[blk] + sl; q < q1; q += kAsmSlices)
-                s += s_contrib(A, A.plan.sblk_src[q], r, c);
-        }
-        if (sl < kAsmSlices) red[sl][e] = s;
+        if (sl < kAsmSlices)
+            red[sl][e] = sum_contribs(
+                A, A.plan.sblk_ptr[g] + sl, A.plan.sblk_ptr[g + 1], kAsmSlices,
+                [&](int q) { return s_contrib(A, A.plan.sblk_src[q], r, c); });
         __syncthreads();
         if (tid < 36) {
             double t = red[0][tid];
@@ -725,21 +758,22 @@ __global__ __launch_bounds__(256) void k_ba_assemble(SolveArgs A) {
             const int row = a * 6 + tid / 6, col = bb * 6 + tid % 6;
             if (row == col) t = t + (double)A.ep + (double)A.lm * t;
             A.S_dbg[(size_t)row * n + col] = t;
+            if (a < bb) A.S_dbg[(size_t)col * n + row] = t;
         }
-    } else {
-        const int a = g - P * P;
+    } else if (g < A.n_blk + P) {
+        const int a = g - A.n_blk;
         const int k = e;  // entries 0..5 of segment a; threads with e >= 6 idle
-        if (sl < kAsmSlices && k < 6) {
-            for (int q = A.plan.bv_ptr[a] + sl; q < A.plan.bv_ptr[a + 1]; q += kAsmSlices) {
-                const int cd = A.plan.bv_src[q];
-                const int v = code_val(cd);
-                if (code_type(cd) == 0)
-                    s += A.etot[(size_t)(v >> 1) * kNT + ((v & 1) ? kTotVj : kTotVi) + k];
-                else
-                    s -= stot_sum(A, (size_t)(A.N_pu + v) * 36 + k);
-            }
-        }
-        if (sl < kAsmSlices) red[sl][e] = s;
+        if (sl < kAsmSlices && k < 6)
+            red[sl][e] = sum_contribs(
+                A, A.plan.bv_ptr[a] + sl, A.plan.bv_ptr[a + 1], kAsmSlices, [&](int q) {
+                    const int cd = A.plan.bv_src[q];
+                    const int v = code_val(cd);
+                    if (code_type(cd) == 0)
+                        return Contrib{A.etot + (size_t)(v >> 1) * kNT +
+                                           ((v & 1) ? kTotVj : kTotVi) + k,
+                                       1, false};
+                    return Contrib{A.stot + (size_t)(A.N_pu + v) * 36 + k, A.nsp, true};
+                });
         __syncthreads();
         if (tid < 6) {
             double t = red[0][tid];
@@ -747,6 +781,15 @@ __global__ __launch_bounds__(256) void k_ba_assemble(SolveArgs A) {
             for (int m = 1; m < kAsmSlices; m++) t += red[m][tid];
             A.b_dbg[a * 6 + tid] = t;
         }
+    } else {
+        const int a = g - A.n_blk - P;
+        for (int col = tid; col < n; col += blockDim.x)
+            if (A.plan.blkmap[a * P + col / 6] < 0) {
+                // the damping of a diagonal block without contributions
+                for (int r = 0; r < 6; r++)
+                    A.S_dbg[(size_t)(a * 6 + r) * n + col] =
+                        a * 6 + r == col ? (double)A.ep : 0.0;
+            }
     }
 }
 
@@ -1316,8 +1359,8 @@ __global__ __launch_bounds__(256) void k_ba_solve_small(SolveArgs A) {
 // r (row 4 r + l / 16, col l % 16)), and a step's product workgroups use no
 // LDS and no barrier.
 // What bounds it: the chain of diagonal blocks (per launch two 64^3 products
-// on one CU's fp64 MFMA, 3.4 us, and the inversion, ~12 us). At n = 1188 a
-// launch takes 22.5 us and the solve 0.48 ms; the Cholesky it replaced, three
+// on one CU's fp64 MFMA, 3.4 us, and the inversion, ~8 us). At n = 1188 a
+// launch takes 18.8 us and the solve 0.39 ms; the Cholesky it replaced, three
 // launches a column (diagonal block in one wave, panel rows one per thread,
 // 64 x 64 update tiles on the vector unit) and the backward solve in one
 // workgroup, took 1.56 ms (17 + 32 + 20 us a column, 258 us backward). Every pivot of the
@@ -1355,83 +1398,85 @@ __device__ __forceinline__ blk_d4 mfma64(double a, double b, blk_d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// v of lane K of this lane's row of 16
-template <int K>
-__device__ __forceinline__ double row16_bcast(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + K, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + K, 0xf, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-
 struct BlkLds {
     double c[2][4][256];  // the waves' blocks of the panel's columns, operand order
     double p[2][256];     // the panel's inverse diagonal block, operand order
-    double m[16][17];     // its unit lower inverse factor
-    double y[16];         // its pivots' reciprocals
     int bad;
 };
 
-// Step K of the elimination of a 16 x 16 block held one row per lane (the
-// four rows of 16 lanes alike): rows below K lose their multiple of row K in
-// every column but K, where the multiple's negative is kept, so columns below
-// the diagonal end as the unit lower L^-1 (its entry (i, K) starts as -f and
-// takes the same updates) and the diagonal as the pivots.
-template <int K, int... Cs>
-__device__ __forceinline__ void blk_elim_step(double (&x)[16], int i16, bool& ok, double& yv,
-                                              std::integer_sequence<int, Cs...>) {
-    const double d = row16_bcast<K>(x[K]);
-    ok = ok && d > 0.0;
-    const double y = rcp_f64(d);
-    yv = i16 == K ? y : yv;
-    const double f = i16 > K ? -(x[K] * y) : 0.0;
-    ((x[Cs] = Cs == K ? (i16 > K ? f : x[Cs])
-                      : __builtin_fma(f, row16_bcast<K>(x[Cs]), x[Cs])),
-     ...);
+// Inverse (i00, i01, i11) of an SPD 2 x 2 block; the determinant's products
+// are compensated. ok: both pivots positive.
+__device__ __forceinline__ void inv2(double a, double b, double c, double& i00, double& i01,
+                                     double& i11, bool& ok) {
+    const double w = b * b, e = __builtin_fma(-b, b, w), det = __builtin_fma(a, c, -w) + e;
+    ok = ok && a > 0.0 && det > 0.0;
+    const double y = rcp_f64(det);
+    i00 = c * y;
+    i01 = -(b * y);
+    i11 = a * y;
 }
-template <int... Ks>
-__device__ __forceinline__ void blk_elim(double (&x)[16], int i16, bool& ok, double& yv,
-                                         std::integer_sequence<int, Ks...>) {
-    (blk_elim_step<Ks>(x, i16, ok, yv, std::make_integer_sequence<int, 16>{}), ...);
+
+// x (an SPD 16 x 16 block, operand order) becomes minus its inverse: a sweep
+// over four panels of 4 columns J. Every lane inverts the 4 x 4 pivot block by
+// 2 x 2 blocks and solves for column g of P = A_JJ^-1; T = C P, x - T C^T and the
+// panel's rows T^T are one product each (a 16 x 16 x 4 product is a panel wide).
+// A chain of 4 x 2 reciprocals; one pivot at a time (16 steps of a reciprocal
+// and 15 row broadcasts) took about 12 us for a 64 x 64 block, about 8 us so.
+__device__ __forceinline__ bool blk_sweep16(double (&x)[4], int lane) {
+    const int i16 = lane & 15, g = lane >> 4;
+    bool ok = true;
+#pragma unroll
+    for (int J = 0; J < 4; J++) {
+        double s[4][4];  // lower triangle
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int b = 0; b <= a; b++) s[a][b] = bcast(x[J], 16 * b + 4 * J + a);
+        double e00, e01, e11, f00, f01, f11;
+        inv2(s[0][0], s[1][0], s[1][1], e00, e01, e11, ok);
+        // H = F E^-1 (rows 2, 3), S = G - H F^T
+        const double h00 = s[2][0] * e00 + s[2][1] * e01, h01 = s[2][0] * e01 + s[2][1] * e11;
+        const double h10 = s[3][0] * e00 + s[3][1] * e01, h11 = s[3][0] * e01 + s[3][1] * e11;
+        inv2(s[2][2] - (h00 * s[2][0] + h01 * s[2][1]), s[3][2] - (h10 * s[2][0] + h11 * s[2][1]),
+             s[3][3] - (h10 * s[3][0] + h11 * s[3][1]), f00, f01, f11, ok);
+        // column g of P
+        const double u0 = g == 0, u1 = g == 1;
+        const double y2 = (g == 2) - (h00 * u0 + h01 * u1), y3 = (g == 3) - (h10 * u0 + h11 * u1);
+        const double p2 = f00 * y2 + f01 * y3, p3 = f01 * y2 + f11 * y3;
+        const double p0 = (e00 * u0 + e01 * u1) - (h00 * p2 + h10 * p3);
+        const double p1 = (e01 * u0 + e11 * u1) - (h01 * p2 + h11 * p3);
+        const double pv = i16 & 2 ? (i16 & 1 ? p3 : p2) : (i16 & 1 ? p1 : p0);
+        const blk_d4 zero = {0.0, 0.0, 0.0, 0.0};
+        const double t = mfma64(pv, x[J], zero)[0];
+        blk_d4 z = {x[0], x[1], x[2], x[3]};
+        z = mfma64(x[J], -t, z);
+        const blk_d4 u = mfma64(t, i16 == 4 * J + g ? 1.0 : 0.0, zero);
+        const bool in = i16 >> 2 == J;
+#pragma unroll
+        for (int q = 0; q < 4; q++) x[q] = q == J ? (in ? -pv : t) : (in ? u[q] : z[q]);
+    }
+    return ok;
 }
 
 // m (this wave's 16 rows of an SPD 64 x 64 block, operand order) becomes its
 // rows of minus the inverse: a block sweep over four 16-column panels. Per
-// panel p every wave publishes its block C of the panel's columns, wave p
-// inverts the diagonal one (P^-1 = L^-T D^-1 L^-1), and with T = C P^-1 every
-// other wave's blocks become m - T C_q^T, its panel block T, and the blocks
-// of wave p P^-1 C_q^T, -P^-1. Two barriers a panel; the buffers alternate.
-// Returns whether every pivot was positive (the same for all threads).
+// panel p every wave publishes its block C of the panel's columns and wave p
+// the diagonal one's inverse P^-1; with T = C P^-1 every other wave's blocks
+// become m - T C_q^T, its panel block T, and the blocks of wave p P^-1 C_q^T,
+// -P^-1. One barrier a panel; the buffers alternate. Returns whether every
+// pivot was positive (the same for all threads).
 __device__ __forceinline__ bool blk_invert(double (&m)[16], BlkLds& L, int wave, int lane) {
-    const int i16 = lane & 15, g = lane >> 4;
     if (threadIdx.x == 0) L.bad = 0;
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         double* c = L.c[p & 1][0];
 #pragma unroll
         for (int r = 0; r < 4; r++) c[wave * 256 + r * 64 + lane] = m[4 * p + r];
-        __syncthreads();
         if (wave == p) {
-            double x[16], yv = 0.0;
-            bool ok = true;
+            double x[4] = {m[4 * p], m[4 * p + 1], m[4 * p + 2], m[4 * p + 3]};
+            if (!blk_sweep16(x, lane)) L.bad = 1;
 #pragma unroll
-            for (int k = 0; k < 16; k++) x[k] = c[p * 256 + (k >> 2) * 64 + (k & 3) * 16 + i16];
-            blk_elim(x, i16, ok, yv, std::make_integer_sequence<int, 16>{});
-            if (g == 0) {
-#pragma unroll
-                for (int k = 0; k < 16; k++) L.m[i16][k] = k < i16 ? x[k] : k == i16 ? 1.0 : 0.0;
-                L.y[i16] = yv;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            blk_d4 pi = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const double t = L.m[4 * s + g][i16];
-                pi = mfma64(t * L.y[4 * s + g], t, pi);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; r++) L.p[p & 1][r * 64 + lane] = pi[r];
-            if (!ok) L.bad = 1;
+            for (int r = 0; r < 4; r++) L.p[p & 1][r * 64 + lane] = -x[r];
         }
         __syncthreads();
         double pinv[4];
@@ -1628,33 +1673,52 @@ __global__ __launch_bounds__(256) void k_blk_step(BlkArgs B, int j) {
             out[trail ? blk_at(wave, 4 * t + r, lane) : blk_at(t, 4 * wave + r, lane)] = acc[t][r];
 }
 
-// x_c = u_c + sum_{i > c} V_ci^T u_i, one workgroup per block column.
+// The terms V_ci^T u_i (i > c) of x_c = u_c + their sum, a workgroup each, into
+// the first row of A_ic, which is not read again. (A workgroup per column
+// streams up to nb - 1 blocks through one compute unit: n = 1188 took 18 us, 5
+// us so.)
 __global__ __launch_bounds__(256) void k_blk_x(BlkArgs B) {
     if (B.flags[2]) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i16 = lane & 15, g = lane >> 4;
-    const int c = blockIdx.x;
-    double s = 0.0;
-#pragma unroll 2
-    for (int i = c + 1; i < B.nb; i++) {
-        const double* v = B.v + blk_idx(i, c);
-        const double* u = B.u + i * kBlk;
-        double e[16], w[16];
+    int i = (int)((sqrtf(8.0f * (float)blockIdx.x + 1.0f) - 1.0f) * 0.5f);
+    while (i > 0 && blk_count(i) > blockIdx.x) i--;
+    while (blk_count(i + 1) <= blockIdx.x) i++;
+    const int c = (int)(blockIdx.x - blk_count(i));
+    i++;  // pair (i, c) of the strict lower triangle
+    const double* v = B.v + blk_idx(i, c);
+    const double* u = B.u + i * kBlk;
+    double e[16], w[16], s = 0.0;
 #pragma unroll
-        for (int k = 0; k < 16; k++) e[k] = v[blk_at(wave, k, lane)];
+    for (int k = 0; k < 16; k++) e[k] = v[blk_at(wave, k, lane)];
 #pragma unroll
-        for (int k = 0; k < 16; k++) w[k] = u[4 * k + g];
+    for (int k = 0; k < 16; k++) w[k] = u[4 * k + g];
 #pragma unroll
-        for (int k = 0; k < 16; k++) s += e[k] * w[k];
-    }
+    for (int k = 0; k < 16; k++) s += e[k] * w[k];
     s += __shfl_xor(s, 16, 64);
     s += __shfl_xor(s, 32, 64);
-    const int row = c * kBlk + wave * 16 + i16;
-    if (g == 0) B.x[row] = s + B.u[row];
+    if (g == 0) B.a[blk_idx(i, c) + wave * 16 + i16] = s;
 }
 
-__global__ __launch_bounds__(256) void k_blk_finish(SolveArgs A, BlkArgs B) {
-    finish_solve(A, B.x, B.flags[2] == 0, solve_halt_word(A), A.poses + 7 * A.t0);
+// x from its terms, then the step (as the other solvers). One workgroup.
+__global__ __launch_bounds__(1024) void k_blk_finish(SolveArgs A, BlkArgs B) {
+    const bool ok = B.flags[2] == 0;
+    if (ok)
+        for (int t = threadIdx.x; t < B.nb * kBlk; t += blockDim.x) {
+            const int c = t / kBlk, k = t % kBlk;
+            double s = 0.0;
+            for (int i = c + 1; i < B.nb; i += 8) {
+                double v[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) v[q] = B.a[blk_idx(min(i + q, B.nb - 1), c) + k];
+#pragma unroll
+                for (int q = 0; q < 8; q++)
+                    if (i + q < B.nb) s += v[q];
+            }
+            B.x[t] = s + B.u[t];
+        }
+    __syncthreads();
+    finish_solve(A, B.x, ok, solve_halt_word(A), A.poses + 7 * A.t0);
 }
 
 // doubles of a solve's working buffer: blocks of S and of L^-1, the diagonal
@@ -1682,8 +1746,9 @@ int solve_blocked(const SolveArgs& A, hipStream_t stream) {
         hipLaunchKernelGGL(k_blk_step, dim3(R * (R + 1) / 2 + R * (j + 1) + 1), dim3(256), 0,
                            stream, B, j);
     }
-    hipLaunchKernelGGL(k_blk_x, dim3(nb), dim3(256), 0, stream, B);
-    hipLaunchKernelGGL(k_blk_finish, dim3(1), dim3(256), 0, stream, A, B);
+    if (nb > 1)
+        hipLaunchKernelGGL(k_blk_x, dim3(nb * (nb - 1) / 2), dim3(256), 0, stream, B);
+    hipLaunchKernelGGL(k_blk_finish, dim3(1), dim3(1024), 0, stream, A, B);
     SLK_HIP(hipGetLastError());
     return SLK_OK;
 }
@@ -3198,7 +3263,7 @@ int iterate_classic(slk_ctx* ctx, BaState* s, const IterArgs& I, hipStream_t str
     const SolveArgs A = solve_args(s, plan, I);
     {
         ProfScope ps(ctx, "ba_assemble", stream);
-        hipLaunchKernelGGL(k_ba_assemble, dim3(s->P * s->P + s->P), dim3(256), 0, stream, A);
+        hipLaunchKernelGGL(k_ba_assemble, dim3(A.n_blk + 2 * s->P), dim3(256), 0, stream, A);
     }
     SLK_HIP(hipGetLastError());
     SLK_TRY(launch_solve(ctx, s, A, stream));

@@ -90,3 +90,34 @@ def test_schur_products_of_many_rows(slk, h, w, hub):
     assert norm_rel(b, ref["b"]) < bound
     assert norm_rel(d["poses"].to_host(), ref["poses"]) < 1e-6
     assert norm_rel(d["disps"].to_host().reshape(-1), ref["disps"].reshape(-1)) < 1e-6
+
+
+def test_system_of_a_sparse_graph_after_a_denser_one(slk):
+    """A chain of 30 keyframes, one of them without edges (an empty diagonal
+    block: only ep there), assembled where a denser graph's system stood: S and
+    b against the oracle, within the products' bound above, and the blocks below
+    the diagonal the exact transposes of those above (inside a diagonal block
+    the entries (r, c) and (c, r) are products of their own)."""
+    orc.build()
+    announce("ba sparse graph after a dense one")
+    n, h, w = 30, 7, 9
+    chain = [(a, b) for a in range(n) for b in (a - 1, a + 1) if 0 <= b < n and 12 not in (a, b)]
+    sparse = wl.ba_problem(n=n, h=h, w=w, ii=np.array([a for a, _ in chain], np.int32),
+                           jj=np.array([b for _, b in chain], np.int32), seed=60)
+    dense = wl.ba_problem(n=n, h=h, w=w, seed=61)
+    ctx, _ = _run(slk, dense, 1e-4, 0.1)
+    d = {k: slk.DeviceArray.from_host(sparse[k])
+         for k in ("poses", "disps", "intr", "target", "weight", "eta", "ii", "jj")}
+    ctx.ba_iterate(d["poses"], d["disps"], d["intr"], d["target"], d["weight"], d["eta"], d["ii"],
+                   d["jj"], sparse["ii"], sparse["jj"], sparse["t0"], sparse["t1"], 1e-4, 0.1)
+    assert ctx.ba_status() == slk.SLK_OK
+    S, b, _ = ctx.ba_last_system()
+    ctx.close()
+    ref = orc.ba_iterate(sparse["poses"], sparse["disps"], sparse["intr"], sparse["target"],
+                         sparse["weight"], sparse["eta"], sparse["ii"], sparse["jj"], h, w,
+                         sparse["t0"], sparse["t1"], 1e-4, 0.1)
+    bound = 4 * h * w * np.finfo(float).eps
+    assert norm_rel(S, ref["S"]) < bound
+    assert norm_rel(b, ref["b"]) < bound
+    off = np.kron(1 - np.eye(len(b) // 6), np.ones((6, 6)))
+    np.testing.assert_array_equal(S * off, S.T * off)
