@@ -700,6 +700,14 @@ __device__ __forceinline__ double sum_contribs(const SolveArgs& A, int q0, int q
                                                int step, const At& at) {
     constexpr int NC = 2;
     double s = 0.0;
+    if (A.nsp == 1) {  // uniform: small systems' lists of edges
+        for (int q = q0; q < q1; q += step) {
+            const Contrib c = at(q);
+            const double t = *c.p;
+            s += c.neg ? -t : t;
+        }
+        return s;
+    }
     for (int q = q0; q < q1; q += NC * step) {
         Contrib c[NC];
         double v[NC][4];
@@ -743,13 +751,14 @@ __global__ __launch_bounds__(256) void k_ba_assemble(SolveArgs A) {
     const int sl = tid / 36, e = tid - sl * 36;
     const int g = blockIdx.x;
     if (g < A.n_blk) {
-        const int ab = A.plan.sblk[g], a = ab / P, bb = ab - a * P;
+        const int ab = A.plan.sblk[g], q0 = A.plan.sblk_ptr[g], q1 = A.plan.sblk_ptr[g + 1];
+        const int a = ab / P, bb = ab - a * P;
         if (a > bb) return;  // the transpose's workgroup writes both
         const int r = e / 6, c = e - r * 6;
         if (sl < kAsmSlices)
-            red[sl][e] = sum_contribs(
-                A, A.plan.sblk_ptr[g] + sl, A.plan.sblk_ptr[g + 1], kAsmSlices,
-                [&](int q) { return s_contrib(A, A.plan.sblk_src[q], r, c); });
+            red[sl][e] = sum_contribs(A, q0 + sl, q1, kAsmSlices, [&](int q) {
+                return s_contrib(A, A.plan.sblk_src[q], r, c);
+            });
         __syncthreads();
         if (tid < 36) {
             double t = red[0][tid];
