@@ -224,7 +224,7 @@ int slk_clamp_disps(float* disps, int n, float min_val, hipStream_t stream);
  * slam::BundleAdjustment::iterate (cuda_pipeline/slam.cuh:1475-1592).
  * One Gauss-Newton step: linearization, Schur complement over the depths of
  * the keyframes in ii (unless motion_only), LM damping S_ii += ep + lm*S_ii,
- * fp64 Cholesky on the GPU, pose retraction of [t0,t1), depth
+ * fp64 LDL^T on the GPU, pose retraction of [t0,t1), depth
  * back-substitution. Stream-ordered and asynchronous (the reference is
  * synchronous); the index structures built from ii_host/jj_host are cached
  * while the edge set is unchanged. An indefinite system leaves poses/disps
