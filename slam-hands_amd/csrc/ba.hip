@@ -3154,6 +3154,7 @@ int ba_prepare(slk_ctx* ctx, const IterArgs& I, const int* ii_host, const int* j
     s->HWs = (HW + 15) / 16 * 16;
     s->nsp = std::max(1, std::min({(4 * s->cus + s->n_zitems - 1) / std::max(1, s->n_zitems),
                                    s->HWs / 128, 8}));
+    if (s->n_zitems == 0) s->nsp = 1;  // motion only: nothing to share, lists of edges
     const size_t pbytes = s->host.size() * sizeof(int);
     SLK_TRY(s->stage.ensure(pbytes));
     std::memcpy(s->stage.ptr, s->host.data(), pbytes);
